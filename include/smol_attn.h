@@ -118,7 +118,7 @@ SMOL_ATTN_API int smol_attn_ctx_timing_read(smol_attn_ctx *ctx, double *ms, int 
 #define SMOL_OPT_DEC_SLABS 3      /* k_dec: 32-key slabs per workgroup (0: by call size) */
 #define SMOL_OPT_DEC_WAVES 4      /* k_dec: 4 or 8 waves per workgroup (0: by shape) */
 #define SMOL_OPT_DEC_SPLIT 5      /* k_dec: -1 keeps every (sequence, kv head) in one workgroup */
-#define SMOL_OPT_XCD_CHECK 6      /* read only: 1 when workgroup b was seen on XCD b % n_xcc at
+#define SMOL_OPT_XCD_CHECK 6      /* read only: 1 when workgroups b and b + n_xcc were seen on one XCD at
                                    * creation (k_dec's split merge needs it), 0 when not (then
                                    * k_dec does not split) */
 #define SMOL_OPT_BIDIR_WIN 7      /* bidirectional windows: 0 (or 1) k_attn_win (LDS-resident,

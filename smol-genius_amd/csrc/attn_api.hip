@@ -199,7 +199,7 @@ struct smol_attn_ctx {
     WinParams wp;
     int cu_count = 256;
     int n_xcc = 1;       /* XCDs of the device */
-    bool xcd_ok = true;  /* workgroup b runs on XCD b % n_xcc (checked at creation) */
+    bool xcd_ok = true;  /* workgroups b and b + n_xcc run on one XCD (checked at creation) */
     unsigned epoch = 0;  /* k_dec launches so far: each one's flags carry its own value */
     int opt[SMOL_OPT_COUNT] = {};
     /* opt-in per-kernel timing: events bracketing each launch */
@@ -311,10 +311,17 @@ static int upload_desc(smol_attn_ctx *ctx, const void *host, size_t bytes) {
 
 /* ------------------------------------------------------------------ context */
 
-/* k_dec merges the splits of a group through one XCD's L2, which needs
- * workgroup b of a launch to run on XCD b % n_xcc (the round-robin dispatch
- * of a device in one partition). A probe grid records each workgroup's XCC
- * id; when any differs, k_dec keeps every group in one workgroup. */
+/* k_dec merges the splits of a group through one XCD's L2, which needs the
+ * workgroups b, b + n_xcc, b + 2 n_xcc ... of a launch to run on one XCD (the
+ * round-robin dispatch of a device in one partition). Which XCD takes
+ * workgroup 0 depends on the stream's hardware queue: of the four queues of
+ * a process one starts at XCD 0, the others at 5, 6 and 7, each always at
+ * the same one, idle or behind other work. So the check is that every
+ * workgroup ran where workgroup b % n_xcc ran, not on XCD b % n_xcc: that
+ * form failed on three streams of four and left their decode calls without
+ * splits (Qwen3-0.6B sizes, 1025 keys: 19.8 us a layer, 12.3 with them). A
+ * probe grid records each workgroup's XCC id; when one differs from its
+ * class, k_dec keeps every group in one workgroup. */
 static int check_xcd_dispatch(smol_attn_ctx *c) {
     int nx = 0;
     if (hipDeviceGetAttribute(&nx, hipDeviceAttributeNumberOfXccs, c->device) != hipSuccess || nx <= 0) nx = 1;
@@ -331,7 +338,7 @@ static int check_xcd_dispatch(smol_attn_ctx *c) {
     hipFree(d);
     if (e != hipSuccess) return fail(SMOL_ATTN_ERR_DEVICE, "XCD probe: %s", hipGetErrorString(e));
     for (int b = 0; b < n; b++)
-        if (h[b] != (unsigned)(b % nx)) c->xcd_ok = false;
+        if (h[b] == 0xFFFFFFFFu || h[b] != h[b % nx]) c->xcd_ok = false;
     return 0;
 }
 

@@ -1115,8 +1115,8 @@ extern "C" int smol_launch_decode(const DecParams *dp, int hd, int rows, int nw,
 
 /* ------------------------------------------------------ XCD dispatch check */
 
-/* workgroup b records the XCC id register; the host checks b % n_xcc, the
- * dispatch order k_dec's merge relies on */
+/* workgroup b records the XCC id register; the host checks that each class
+ * b % n_xcc ran on one XCD, the dispatch order k_dec's merge relies on */
 __global__ __launch_bounds__(64) void k_xcc_probe(unsigned *out, int n) {
     unsigned x;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));

@@ -189,7 +189,7 @@ typedef struct {
     int tpu;                   /* tiles of the longest window */
     int ksplit;                /* 1: a workgroup's 8 waves hold 128 rows over every key; 2: two groups of
                                   4 waves hold 64 rows, each over half the window's slabs, merged in LDS */
-    int n_xcc;                 /* XCDs: workgroup b runs on XCD b % n_xcc */
+    int n_xcc;                 /* XCDs: workgroups b and b + n_xcc run on one XCD */
     int *range_flag;           /* set to 1 when a value written as fp16 would overflow */
     int precise;               /* 1: QK^T on fp16 hi + lo operands (Q always; K for fp32 inputs) */
     int ws[WIN_ARG_WINDOWS + 1];
@@ -200,7 +200,7 @@ typedef struct {
  * A group is one (sequence, kv head): its R = n_q * G query rows (R <= 64)
  * against the sequence's keys, split into n_split contiguous slab ranges,
  * one workgroup each. Every workgroup of a group runs on the same XCD
- * (workgroup b runs on XCD b % n_xcc, checked when a context is created), so
+ * (workgroups b and b + n_xcc do, checked when a context is created), so
  * the partials and flags of a group meet in that XCD's L2. There is no
  * atomic: each split publishes its partial, waits for the stores, then
  * writes the call's epoch into its flag; the group's last split, placed

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(WIN_TPB) void k_attn_win(const WinParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     /* Unit u = (window u / H, head u % H) has up to tpu tiles of WIN_ROWS. The
      * units go round-robin over the XCDs and a unit's tiles to one XCD
-     * (workgroup b runs on XCD b % n_xcc), so the window's K and V come
+     * (workgroups b and b + n_xcc do), so the window's K and V come
      * from memory into one L2 and its tiles share them there. */
     const int b = blockIdx.x, nx = p.n_xcc;
     const int x = b % nx, slot = b / nx;

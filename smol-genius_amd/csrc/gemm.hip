@@ -34,8 +34,8 @@
  * stages in flight while one is multiplied. LDS rows are 128 or 256 bytes
  * with their 16-byte chunks XOR-swizzled by the row's low 3 bits, so the
  * fragment reads of eight consecutive lanes hit distinct banks. The tile
- * grid is cut into eight regions, one per XCD (workgroup b runs on XCD
- * b % 8), shaped to keep the fewest x and W bytes per XCD L2.
+ * grid is cut into eight regions, one per XCD (workgroups b and b + 8 run on
+ * one XCD), shaped to keep the fewest x and W bytes per XCD L2.
  */
 #include "attn_device.h"
 #include "smol_linear.h"
@@ -121,7 +121,7 @@ void k_gemm(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[NSTG * STAGE];
     __shared__ float s_rinv[NORM ? BM : 1];
 
-    /* the tile: workgroup b runs on XCD b % 8 */
+    /* the tile: workgroups b and b + 8 run on one XCD */
     const int b = blockIdx.x, xcd = b % GEMM_XCD, idx = b / GEMM_XCD;
     int tm, tn;
     if (p.rm > 0) {

@@ -790,3 +790,28 @@ def test_decode_merge_timeout_reported(ctx, sa, oracle, wo, opts):
     r.step()
     ctx.synchronize()  # the flag was cleared by the failed synchronize
     assert_parity(r.outputs(), wo.decode(oracle, wl, x), "decode after a timed-out merge")
+
+
+def test_decode_split_on_every_stream(sa, oracle, wo):
+    """The split merge is available whatever hardware queue a context's
+    stream runs on (the queues start their round robin at different XCDs),
+    and decode on each stream meets the oracle."""
+    from smol_genius_amd import runner
+    from smol_genius_amd.workloads import Decode
+    wl = Decode("t", 16, 8, 128, [1025], 1e6, 0, seed=190)
+    x = wl.inputs()
+    want = wo.decode(oracle, wl, x)
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    for i, st in enumerate(streams):
+        print("decode split stream", i, flush=True)
+        torch.cuda.synchronize()
+        c = sa.Context(0, st.cuda_stream)
+        try:
+            assert c.get_option(sa.OPT_XCD_CHECK) == 1
+            r = runner.prepare(c, wl, x)
+            torch.cuda.synchronize()
+            r.step()
+            c.synchronize()
+            assert_parity(r.outputs(), want, "decode on stream %d" % i)
+        finally:
+            c.close()
