@@ -272,7 +272,8 @@ typedef struct {
     DecItem items[DEC_ARG_ITEMS];
 } DecParams;
 
-/* ---- k_gemm (gemm.hip): the projections on bf16 MFMA ---- */
+/* ---- k_gemm (gemm.hip) and k_gemm_kw (gemm_kw.hip): the projections on bf16 MFMA ---- */
+#define GEMM_CFGS 9 /* tile configurations of both (smol_gemm_tile) */
 struct GemmParams {
     const uint16_t *w; /* [N][K] bf16 */
     const void *x;     /* [M][K] fp32 or bf16 */

@@ -37,11 +37,9 @@
  * grid is cut into eight regions, one per XCD (workgroups b and b + 8 run on
  * one XCD), shaped to keep the fewest x and W bytes per XCD L2.
  */
-#include "attn_device.h"
-#include "smol_linear.h"
+#include "gemm_device.h"
 
 #define GEMM_BK 64
-#define GEMM_XCD 8
 
 
 namespace {
@@ -71,40 +69,6 @@ __device__ __forceinline__ unsigned swz(int row, int q, int rb) {
     return (unsigned)(row * rb + ((q ^ (row & 7)) << 4));
 }
 
-__device__ __forceinline__ float act_fn(float g, int act) {
-    if (act == SMOL_LINEAR_ACT_SWIGLU) return g / (1.0f + expf(-g));
-    const float x3 = g * g * g;
-    const float inner = 0.7978845608028654f * (g + 0.044715f * x3);
-    return 0.5f * g * (1.0f + tanhf(inner));
-}
-
-/* x_hi = bf16_rne(x), x_lo = bf16_rne(xc - bf16_rne(xc)) of 8 floats, xc =
- * x clamped to bf16's largest finite magnitude (about 3.39e38): the same
- * x_lo for every |x| up to that bound, 0 for an infinite x (which goes to
- * x_hi whole and so reaches y as it would in fp32), never an infinite or
- * NaN lo part beside a finite one. Per pair: one packed conversion for the
- * hi pair, two clamps, two conversions over a zero low half (which are
- * bf16(xc) as floats), two differences, one packed conversion for the lo
- * pair. */
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float fl2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_frag(const float *v, b8 &hi, b8 &lo) {
-    constexpr float BF16_MAX = 3.3895313892515355e38f;
-    uint32_t hw[4], lw[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float x0 = v[2 * i], x1 = v[2 * i + 1];
-        hw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((fl2){x0, x1}, bf2));
-        const float c0 = __builtin_amdgcn_fmed3f(x0, -BF16_MAX, BF16_MAX);
-        const float c1 = __builtin_amdgcn_fmed3f(x1, -BF16_MAX, BF16_MAX);
-        const float h0 = __builtin_bit_cast(float, __builtin_convertvector((fl2){0.0f, c0}, bf2));
-        const float h1 = __builtin_bit_cast(float, __builtin_convertvector((fl2){0.0f, c1}, bf2));
-        lw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((fl2){c0 - h0, c1 - h1}, bf2));
-    }
-    hi = as_b8(make_uint4(hw[0], hw[1], hw[2], hw[3]));
-    lo = as_b8(make_uint4(lw[0], lw[1], lw[2], lw[3]));
-}
-
 } // namespace
 
 template <int BM, int BN, int WN, int WM, bool XBF, bool YBF, bool NORM>
@@ -121,40 +85,13 @@ void k_gemm(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[NSTG * STAGE];
     __shared__ float s_rinv[NORM ? BM : 1];
 
-    /* the tile: workgroups b and b + 8 run on one XCD */
-    const int b = blockIdx.x, xcd = b % GEMM_XCD, idx = b / GEMM_XCD;
     int tm, tn;
-    if (p.rm > 0) {
-        /* XCD x: region (x / rn, x % rn) of the tile grid, so the rows of x
-         * and of W that its tiles share stay in its own L2 */
-        const int tiles_n = p.tiles / p.tiles_m;
-        const int ri = xcd / p.rn, rj = xcd % p.rn;
-        const int m_lo = ri * p.tiles_m / p.rm, m_hi = (ri + 1) * p.tiles_m / p.rm;
-        const int n_lo = rj * tiles_n / p.rn, n_hi = (rj + 1) * tiles_n / p.rn;
-        if (idx >= (m_hi - m_lo) * (n_hi - n_lo)) return;
-        tm = m_lo + idx % (m_hi - m_lo);
-        tn = n_lo + idx / (m_hi - m_lo);
-    } else {
-        const int t = xcd * p.per_xcd + idx;
-        if (idx >= p.per_xcd || t >= p.tiles) return;
-        tm = t % p.tiles_m;
-        tn = t / p.tiles_m;
-    }
+    if (!gemm_tile_of(p, blockIdx.x, tm, tn)) return;
     const int m0 = tm * BM;
     const int K = p.K;
-    /* the tile's output: its segment's weight rows, y and width (a tile
-     * never straddles two segments) */
-    int n0 = tn * BN, NN = p.N;
-    const uint16_t *Wt = p.w;
-    void *Yt = p.y;
-    if (p.nseg > 0) {
-        const int sg = (n0 >= p.seg_c[1] ? 1 : 0) + (p.nseg > 2 && n0 >= p.seg_c[2] ? 1 : 0);
-        const int c0 = sg == 0 ? 0 : sg == 1 ? p.seg_c[1] : p.seg_c[2];
-        NN = (sg == 0 ? p.seg_c[1] : sg == 1 ? p.seg_c[2] : p.seg_c[3]) - c0;
-        Wt = sg == 0 ? p.seg_w[0] : sg == 1 ? p.seg_w[1] : p.seg_w[2];
-        Yt = sg == 0 ? p.seg_y[0] : sg == 1 ? p.seg_y[1] : p.seg_y[2];
-        n0 -= c0;
-    }
+    const GemmOut out = gemm_out_of(p, tn * BN);
+    const int n0 = out.n0, NN = out.n;
+    const uint16_t *Wt = out.w;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -346,8 +283,6 @@ void k_gemm(const GemmParams p) {
 
     /* epilogue: lane (c, j) holds outputs n = 4 j + e of row m = c of each
      * 16 x 16 product tile */
-    const bool has_act = p.act != SMOL_LINEAR_ACT_NONE;
-    const int ycols = has_act ? NN / 2 : NN;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const int ml = wm * Gm::TM + 16 * mt + c;
@@ -359,57 +294,15 @@ void k_gemm(const GemmParams p) {
             const int n = n0 + wn * Gm::TN + 16 * t + 4 * j;
             if (n >= NN) continue;
             float v[4] = {acc[t][mt][0], acc[t][mt][1], acc[t][mt][2], acc[t][mt][3]};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (NORM) v[e] *= r;
-                if (p.bias) v[e] += n + e < NN ? p.bias[n + e] : 0.0f;
-            }
-            if (has_act) {
-                const int col = n / 2;
-                float o[2] = {act_fn(v[0], p.act) * v[1], act_fn(v[2], p.act) * v[3]};
-                const long long yi = (long long)m * ycols + col;
-                const int nv = min(2, ycols - col);
-                if (p.res) {
-#pragma unroll
-                    for (int e = 0; e < 2; e++)
-                        if (e < nv) o[e] += p.res[yi + e];
-                }
-                if constexpr (YBF) {
-                    uint16_t *y = static_cast<uint16_t *>(Yt) + yi;
-#pragma unroll
-                    for (int e = 0; e < 2; e++)
-                        if (e < nv) y[e] = (uint16_t)(__float_as_uint(o[e]) >> 16);
-                } else {
-                    float *y = static_cast<float *>(Yt) + yi;
-                    if (nv == 2 && ((yi & 1) == 0)) *reinterpret_cast<float2 *>(y) = make_float2(o[0], o[1]);
-                    else
-                        for (int e = 0; e < nv; e++) y[e] = o[e];
-                }
-            } else {
-                const long long yi = (long long)m * ycols + n;
-                const int nv = min(4, NN - n);
-                if (p.res) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (e < nv) v[e] += p.res[yi + e];
-                }
-                if constexpr (YBF) {
-                    uint16_t *y = static_cast<uint16_t *>(Yt) + yi;
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (e < nv) y[e] = (uint16_t)(__float_as_uint(v[e]) >> 16);
-                } else {
-                    float *y = static_cast<float *>(Yt) + yi;
-                    if (nv == 4 && ((yi & 3) == 0)) *reinterpret_cast<float4 *>(y) = make_float4(v[0], v[1], v[2], v[3]);
-                    else
-                        for (int e = 0; e < nv; e++) y[e] = v[e];
-                }
-            }
+            gemm_store4<YBF, NORM>(p, out.y, m, n, NN, v, r);
         }
     }
 }
 
 /* ------------------------------------------------------------------ launch */
+
+extern "C" int smol_launch_gemm_kw(const GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
+                                   hipEvent_t e1);
 
 template <int BM, int BN, int WN, int WM, bool XBF, bool YBF>
 static int launch_gemm_t(const GemmParams &p, bool norm, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
@@ -441,10 +334,13 @@ static int launch_gemm_b(const GemmParams &p, bool xbf, bool ybf, bool norm, hip
                : launch_gemm_t<BM, BN, WNF, WMF, false, false>(p, norm, st, e0, e1);
 }
 
-/* tile sizes the host may choose (rows of x = BM, outputs = BN) */
+/* the configurations the host may choose (rows of x = BM, outputs = BN):
+ * 0-2 k_gemm, 3-8 k_gemm_kw (gemm_kw.hip), of which 4 and 6 split K over four
+ * waves and the others over eight */
 extern "C" int smol_gemm_tile(int cfg, int *bm, int *bn) {
-    static const int t[3][2] = {{192, 192}, {128, 128}, {64, 64}};
-    if (cfg < 0 || cfg > 2) return -1;
+    static const int t[GEMM_CFGS][2] = {{192, 192}, {128, 128}, {64, 64}, {64, 64}, {64, 64},
+                                        {32, 64},   {32, 32},   {16, 32}, {16, 16}};
+    if (cfg < 0 || cfg >= GEMM_CFGS) return -1;
     *bm = t[cfg][0];
     *bn = t[cfg][1];
     return 0;
@@ -486,6 +382,7 @@ extern "C" int smol_launch_gemm(GemmParams *p, int cfg, bool xbf, bool ybf, hipS
     } else {
         p->per_xcd = (p->tiles + GEMM_XCD - 1) / GEMM_XCD;
     }
+    if (cfg > 2) return smol_launch_gemm_kw(p, cfg, xbf, ybf, st, e0, e1);
     const bool norm = p->g != nullptr;
     switch (cfg) {
     case 0: return launch_gemm_b<192, 192, 2, 4, 2, 4>(*p, xbf, ybf, norm, st, e0, e1);

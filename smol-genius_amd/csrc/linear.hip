@@ -20,7 +20,8 @@
  *            step is issued before the first FMA. Sums: per-lane fp32, then
  *            a wave all-reduce (cross-row swaps + DPP row rotations), then
  *            the kp waves' totals in a fixed order through LDS.
- *   k_gemm   longer inputs (gemm.hip): bf16 MFMA tiles with the input
+ *   k_gemm   longer inputs (gemm.hip; gemm_kw.hip for a few to a few
+ *            hundred rows): bf16 MFMA tiles with the input
  *            RMSNorm, the bias, the gated activation and the residual add
  *            fused; an fp32 x is split into bf16 hi + lo as it is staged
  *            (y = W x_hi + W x_lo, x carried to ~2^-17 relative, the
@@ -728,18 +729,37 @@ int run_gemv_rows(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const v
     return 0;
 }
 
-/* k_gemm's tile configurations (gemm.hip): 192 x 192, 128 x 128 and 64 x 64
- * (rows x outputs); one workgroup per compute unit for the first two, two
- * for the last. The time of a launch is about its rounds of workgroups over
- * the device times a round's time; the weights below are the measured time
- * of one round per unit of tile area relative to 192 x 192 (M = 1536,
- * K = 1024, fp32 x: about 41-51, 22-24 and 16-18 us a round; the bf16 x
- * ratios are alike). */
-int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int seg_align = 0) {
-    static const int per_cu[3] = {1, 1, 2};
-    static const float cost[3] = {1.0f, 1.15f, 3.4f};
+/* The configuration for an M x N product over K (smol_gemm_tile): the one
+ * of least estimated time. With R rounds of workgroups over the device (one
+ * workgroup per compute unit a round; two of k_gemm's 64 x 64, which are
+ * resident together) a launch takes about
+ *     a + R (b + c K) + d (weight MB)   us,
+ * K in thousands, rounded up to what the waves split it into. The constants
+ * are fitted (least squares of the relative error) to the measured times of
+ * every configuration at 8 to 1536 rows, 1024 to 12288 outputs and K = 1024
+ * to 6144, weights not in L2; there the choice is within 1.5% of the best
+ * configuration on average, 33% at worst (700 bf16 rows, 1024 -> 6144), and
+ * within 4% of the best k_gemm tile everywhere. Where the lines fall: for
+ * K = 1024, N = 1024 k_gemm_kw up to about 700 rows, for N = 6144 up to about
+ * 128. */
+int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, int seg_align = 0) {
+    struct Cost {
+        int per_cu, kstep; /* workgroups per compute unit; K of one step of all its waves */
+        float f32[4], bf16[4];
+    };
+    static const Cost cost[GEMM_CFGS] = {
+        {1, 64, {0.00f, 9.66f, 26.07f, 0.523f}, {0.00f, 6.63f, 14.06f, 0.003f}},
+        {1, 64, {0.00f, 6.21f, 13.45f, 0.257f}, {0.00f, 5.07f, 9.75f, 0.00f}},
+        {2, 64, {0.00f, 4.69f, 7.37f, 0.121f}, {0.00f, 2.82f, 6.94f, 0.049f}},
+        {1, 256, {0.00f, 6.35f, 4.40f, 0.075f}, {1.50f, 3.71f, 3.42f, 0.035f}},
+        {1, 128, {3.53f, 2.49f, 5.30f, 0.091f}, {3.42f, 1.26f, 3.44f, 0.024f}},
+        {1, 256, {0.466f, 4.68f, 2.95f, 0.078f}, {2.27f, 2.39f, 2.71f, 0.048f}},
+        {1, 256, {3.85f, 1.22f, 2.11f, 0.085f}, {3.76f, 0.571f, 1.28f, 0.038f}},
+        {1, 512, {1.54f, 3.23f, 1.23f, 0.094f}, {2.72f, 2.12f, 0.850f, 0.066f}},
+        {1, 512, {2.68f, 2.21f, 0.782f, 0.107f}, {3.23f, 1.15f, 0.530f, 0.041f}},
+    };
     const int forced = smol_internal_ctx_option(ctx, SMOL_OPT_GEMM_TILE);
-    if (forced >= 1 && forced <= 3) {
+    if (forced >= 1 && forced <= GEMM_CFGS) {
         int bm, bn;
         smol_gemm_tile(forced - 1, &bm, &bn);
         return seg_align % bn == 0 ? forced - 1 : -1;
@@ -747,13 +767,17 @@ int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int seg_align = 0) {
     const int cus = smol_internal_ctx_cus(ctx);
     int best = -1;
     double best_t = 1e300;
-    for (int cfg = 0; cfg < 3; cfg++) {
+    for (int cfg = 0; cfg < GEMM_CFGS; cfg++) {
         int bm, bn;
         smol_gemm_tile(cfg, &bm, &bn);
         if (seg_align % bn != 0) continue; /* segment boundaries on tile edges */
+        const Cost &q = cost[cfg];
+        const float *f = xbf ? q.bf16 : q.f32;
         const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const long long slots = (long long)cus * per_cu[cfg];
-        const double t = (double)((tiles + slots - 1) / slots) * bm * bn * cost[cfg];
+        const long long slots = (long long)cus * q.per_cu;
+        const double rounds = (double)((tiles + slots - 1) / slots);
+        const double k = (double)((K + q.kstep - 1) / q.kstep) * q.kstep / 1024;
+        const double t = f[0] + rounds * (f[1] + k * f[2]) + f[3] * ((double)N * K * 2e-6);
         if (t < best_t) {
             best_t = t;
             best = cfg;
@@ -787,7 +811,7 @@ int run_gemm(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const void *
     p.rm = 1; /* the launcher chooses the region split */
     hipEvent_t e0 = nullptr, e1 = nullptr;
     smol_internal_timing_events(ctx, LIN_TIMING_KIND, &e0, &e1);
-    const int rc = smol_launch_gemm(&p, gemm_cfg(ctx, seq, out), xbf, ybf, st, e0, e1);
+    const int rc = smol_launch_gemm(&p, gemm_cfg(ctx, seq, out, in, xbf), xbf, ybf, st, e0, e1);
     if (rc) return lfail(SMOL_ATTN_ERR_DEVICE, rc == -1 ? "k_gemm: unsupported operands" : "k_gemm launch failed");
     return 0;
 }
@@ -804,7 +828,7 @@ int run_gemm_qkv(smol_attn_ctx *ctx, hipStream_t st, void *q, void *k, void *v, 
         (f && f->norm_w && !aligned16(f->norm_w)) || (long long)q_dim * in * 2 > 0x7FFF0000LL ||
         (long long)kv_dim * in * 2 > 0x7FFF0000LL || (long long)seq * in * 4 > 0x7FFF0000LL)
         return 1;
-    const int cfg = gemm_cfg(ctx, seq, q_dim + 2 * kv_dim, std::gcd(q_dim, kv_dim));
+    const int cfg = gemm_cfg(ctx, seq, q_dim + 2 * kv_dim, in, xbf, std::gcd(q_dim, kv_dim));
     if (cfg < 0) return 1;
     GemmParams p{};
     p.w = wq;

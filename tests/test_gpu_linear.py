@@ -250,6 +250,52 @@ def test_gemm_every_tile(ctx, sa, oracle, tile):
         ctx.set_option(sa.OPT_GEMM_TILE, 0)
 
 
+@pytest.mark.parametrize("tile", range(4, 10), ids=["64x64_8", "64x64_4", "32x64_8", "32x32_4", "16x32_8", "16x16_8"])
+def test_gemm_k_over_waves(ctx, sa, oracle, tile):
+    """k_gemm_kw's configurations forced, at the sizes where they can go wrong:
+    K below one step, not a multiple of a step or of all the waves' steps, and
+    more steps than a wave holds in flight; rows and outputs one past a tile;
+    Q, K and V as segments; the fused norm, activation and residual."""
+    ctx.set_option(sa.OPT_GEMM_TILE, tile)
+    try:
+        for seq, n_in, n_out, has_b, xbf, ybf in [(5, 8, 17, True, False, False), (17, 40, 16, False, True, False),
+                                                  (33, 520, 65, True, False, True), (65, 1000, 390, False, False, False),
+                                                  (64, 3072, 130, True, True, True), (129, 2048, 64, False, False, False)]:
+            print("gemm kw", tile, seq, n_in, n_out, xbf, ybf, flush=True)
+            x, w, b = linear_inputs(8700 + n_in + n_out + tile, seq, n_in, n_out, has_b)
+            if xbf:
+                xbits = synth.f32_to_bf16_bits(x)
+                x = synth.bf16_bits_to_f32(xbits)
+                xd = dev_bits(xbits).view(torch.bfloat16)
+            else:
+                xd = dev(x)
+            y = sa.linear(ctx, xd, dev_bits(w), dev(b) if has_b else None, out_bf16=ybf)
+            ctx.synchronize()
+            ref = oracle.linear_bf16(x, w, b)
+            if ybf:  # truncated: one bf16 step below
+                g = synth.bf16_bits_to_f32(y.cpu().numpy().view(np.uint16)).astype(np.float64)
+                assert (np.abs(g - ref) <= np.abs(ref) * 2.0 ** -7 + bound(x, w, b)).all()
+            else:
+                check(y.cpu().numpy(), ref, x, w, b, "gemm kw %d %s" % (tile, (seq, n_in, n_out)))
+        seq, n_in, n_out = 37, 1000, 392
+        x, w, b = linear_inputs(8800 + tile, seq, n_in, n_out, True)
+        g = (1.0 + 0.1 * synth.normal(8801, (n_in,))).astype(np.float32)
+        r = synth.normal(8802, (seq, n_out // 2))
+        xn = oracle.rms_norm(x, g, 1e-6)
+        ref = (r.astype(np.float64) + oracle.glu(oracle.linear_bf16(xn, w, b), 1)).astype(np.float32)
+        rd = dev(r)
+        sa.linear_ops(ctx, dev(x), dev_bits(w), dev(b), norm_weight=dev(g), eps=1e-6, act=1, residual=rd, out=rd)
+        ctx.synchronize()
+        assert_parity(rd.cpu().numpy(), ref, "gemm kw %d ops" % tile)
+        ws = [linear_inputs(8810 + i, seq, n_in, n, False)[1] for i, n in enumerate((192, 64, 64))]
+        got = sa.linear_qkv_norm(ctx, dev(x), *[dev_bits(v) for v in ws], dev(g), 1e-6)
+        ctx.synchronize()
+        for y, v in zip(got, ws):
+            assert_parity(y.cpu().numpy(), oracle.linear_bf16(xn, v), "gemm kw %d qkv" % tile)
+    finally:
+        ctx.set_option(sa.OPT_GEMM_TILE, 0)
+
+
 def test_gemm_full_prefill_shapes(ctx, sa, oracle):
     """Qwen3-0.6B projections of a 1536-token prefill: sampled rows against the
     oracle, every row against a float64 product on the device."""
