@@ -135,9 +135,9 @@ SMOL_ATTN_API int smol_attn_ctx_timing_read(smol_attn_ctx *ctx, double *ms, int 
 #define SMOL_OPT_QK_FP16 11       /* 1: QK^T on single fp16 operands (Q and K each rounded to fp16:
                                    * faster, within the bar for logits up to about sigma 1.4 on
                                    * unit-variance rows); 0: fp16 hi + lo operands, see Numerics */
-#define SMOL_OPT_FB_GROUPS 12     /* k_attn_fb: 1: one key group of eight waves over 128-row items (long
-                                   * items' keys split over workgroups and merged); 0 or 2: two key
-                                   * groups over 64-row items */
+#define SMOL_OPT_FB_GROUPS 12     /* k_attn_fb at head_dim <= 128: 0: chosen per call; 1: one key group of
+                                   * eight waves over 128-row items (long items' keys split over workgroups
+                                   * and merged); 2: two key groups over 64-row items */
 #define SMOL_OPT_GEMM_TILE 13     /* k_gemm (projections of more than 4 rows): 0: tile chosen per shape;
                                    * 1, 2, 3: 192 x 192, 128 x 128, 64 x 64 (rows x outputs); 4 to 9: K split
                                    * over the waves of a workgroup, 64 x 64 over eight and over four, 32 x 64

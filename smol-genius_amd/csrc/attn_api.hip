@@ -39,6 +39,8 @@ extern "C" int smol_launch_xcc_probe(unsigned *out, int n, hipStream_t st);
 extern "C" int smol_decode_occupancy(int hd, int rows, int nw, int direct);
 extern "C" int smol_launch_fa(const SkParams *sp, int hd, int n_items, int nt, int w, hipStream_t st, hipEvent_t ev0,
                               hipEvent_t ev1);
+extern "C" int smol_launch_sk_merge(const SkParams *sp, const SkMerge *groups, int n, int rows, int hd,
+                                    hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 extern "C" int smol_launch_fb(const SkParams *sp, int hd, int n_items, int nt, hipStream_t st, hipEvent_t ev0,
                               hipEvent_t ev1);
 extern "C" int smol_launch_win(const WinParams *wp, int hd, int n_tiles, int max_len, hipStream_t st, hipEvent_t e0,
@@ -183,7 +185,7 @@ struct smol_attn_ctx {
     int ring_next = 0;
     DevBuf desc;   /* device copy of the descriptor tables */
     std::vector<unsigned char> desc_last; /* host bytes of the last upload to `desc` */
-    DevBuf qs, kf, vtf, part_o, part_ml, counters;
+    DevBuf qs, kf, vtf, part_o, part_ml;
     DevBuf kf_lo; /* fp16 lo part of the fresh K (precise QK^T) */
     DevBuf qs32; /* fp32 Q scratch of the decode kernel */
     DevBuf out32; /* fp32 result of a call whose output is bf16 */
@@ -382,7 +384,7 @@ extern "C" int smol_attn_ctx_destroy(smol_attn_ctx *ctx) {
     if (!ctx) return SMOL_ATTN_OK;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
-    DevBuf *bufs[] = {&ctx->desc, &ctx->qs, &ctx->kf, &ctx->kf_lo, &ctx->vtf, &ctx->part_o, &ctx->part_ml, &ctx->counters,
+    DevBuf *bufs[] = {&ctx->desc, &ctx->qs, &ctx->kf, &ctx->kf_lo, &ctx->vtf, &ctx->part_o, &ctx->part_ml,
                       &ctx->qs32, &ctx->out32, &ctx->dec_part};
     for (DevBuf *b : bufs)
         if (b->p) hipFree(b->p);
@@ -707,9 +709,23 @@ static void plan_items(Plan &pl, int Hkv, int G, int window, int rows_per, int c
     long long per = (total_slabs * Hkv + target_items - 1) / std::max(1LL, target_items);
     /* k_attn_fa gives each slab to all four waves: at least four slabs per item */
     int slabs_per_item = (int)std::max(4LL, per);
-    if (no_split) slabs_per_item = 1 << 28;
+    if (no_split) {
+        slabs_per_item = 1 << 28;
+    } else if ((long long)tiles.size() * Hkv <= target_items) {
+        /* each tile rounds its pieces up: longer pieces until they fit the
+         * device in one round (a second round of a few workgroups took as
+         * long as the first: 1000 rows on 2548 keys, 544 workgroups for 512
+         * places, 69.6 us; 512, 53) */
+        auto pieces = [&](int per_item) {
+            long long n = 0;
+            for (const Tile &t : tiles)
+                n += std::max(1, ((t.hi - t.lo + SMOL_SLAB - 1) / SMOL_SLAB + per_item - 1) / per_item);
+            return n * Hkv;
+        };
+        while (pieces(slabs_per_item) > target_items) slabs_per_item++;
+    }
     int group = 0;
-    const int max_split = SK_MERGE_MAX / rows_per; /* the kernel's merge holds rows * n_split pairs in LDS */
+    const int max_split = SK_MAX_SPLIT;
     for (const Tile &t : tiles) {
         const int n_slabs = (t.hi - t.lo + SMOL_SLAB - 1) / SMOL_SLAB;
         int want = std::max(1, (n_slabs + slabs_per_item - 1) / slabs_per_item);
@@ -734,19 +750,27 @@ static void plan_items(Plan &pl, int Hkv, int G, int window, int rows_per, int c
     pl.n_groups = group;
 }
 
-/* k_attn_fb with one key group: 128-row tiles cut into key pieces that fill
- * each workgroup's list to the same cost. The tiles, largest first, are laid
- * into lists of capacity C in turn, a tile cut exactly where a list is full
- * and continued in the next; a piece costs its slabs plus `overhead` steps
- * (start-up, epilogue, and a publish / merge when the tile is cut), and C is
- * the total cost over the workgroups a kv head gets (raised until the lists
- * fit). The pieces of a tile merge (group = tile, partial slots contiguous);
- * pl.items holds the pieces in slot order and `lists` each list's pieces. */
-static void plan_fb_fill(Plan &pl, int Hkv, int G, int window, int cu_count, std::vector<std::vector<int>> &lists) {
-    const int rows_per = 128, overhead = 3;
+/* k_attn_fb with one key group: the tiles (rows_per rows) cut into key
+ * pieces, each a work item; the pieces of a tile merge (group = tile, partial
+ * slots contiguous). pl.items holds the pieces in slot order, `lists` the
+ * pieces of each workgroup of a kv head.
+ *
+ * Fewer tiles than workgroups: each tile is cut into equal pieces, one a
+ * workgroup, as long as shorter pieces gain more than the longer merge costs
+ * (a step of the slab loop against 0.1 steps a piece, and three for writing
+ * partials and the merge's launch). Otherwise the tiles, largest first, are laid into lists
+ * of capacity C in turn, a tile cut exactly where a list is full and
+ * continued in the next; a piece costs its slabs plus `overhead` steps
+ * (start-up, epilogue), and C is the total cost over the workgroups (raised
+ * until the lists fit). Returns the steps that two-group items (64 rows, two
+ * slabs a step) of the call would take. */
+static double plan_fb_one(Plan &pl, int Hkv, int G, int window, int rows_per, int cu_count,
+                        std::vector<std::vector<int>> &lists) {
+    const int overhead = 3;
     struct Tile { int batch, row0, lo, hi, n; };
     std::vector<Tile> tiles;
     long long total = 0;
+    int longest = 1;
     for (int bi = 0; bi < (int)pl.sb.size(); bi++) {
         const SkBatch &b = pl.sb[bi];
         for (int r0 = 0; r0 < b.n_rows; r0 += rows_per) {
@@ -760,61 +784,79 @@ static void plan_fb_fill(Plan &pl, int Hkv, int G, int window, int cu_count, std
             const int n = hi > lo ? (hi - lo + SMOL_SLAB - 1) / SMOL_SLAB : 0;
             tiles.push_back({bi, r0, lo, std::max(hi, lo), n});
             total += n + overhead;
+            longest = std::max(longest, n);
         }
     }
     std::stable_sort(tiles.begin(), tiles.end(), [](const Tile &a, const Tile &b) { return a.n > b.n; });
-    const int n_wg = std::max(1, cu_count / std::max(1, Hkv));
-    const int max_split = SK_MERGE_MAX / rows_per;
+    const int per = std::max(1, cu_count / std::max(1, Hkv)); /* workgroups of a kv head */
+    const double two = std::max(longest / 2.0, (double)total / (rows_per / 64) / per);
+    const int n_tiles = (int)tiles.size();
     struct Piece { int tile, first, count; };
     std::vector<std::vector<Piece>> bins;
-    for (double cap = std::max(1.0, (double)total / n_wg);; cap *= 1.02) {
-        bins.assign(1, {});
-        double room = cap;
-        bool ok = true;
-        for (int t = 0; t < (int)tiles.size() && ok; t++) {
-            int first = 0, made = 0;
-            do {
-                if (room < overhead + 1 && !bins.back().empty()) {
-                    bins.push_back({});
-                    room = cap;
-                }
-                const int left = tiles[t].n - first;
-                const int take = std::min(left, std::max(1, (int)(room - overhead)));
-                bins.back().push_back({t, first, take});
-                first += take;
-                room -= take + overhead;
-                if (++made > max_split) ok = false;
-            } while (first < tiles[t].n);
+    if (n_tiles <= per) {
+        int best = longest;
+        double best_c = longest;
+        for (int len = longest - 1; len >= 1; len--) {
+            long long n = 0;
+            for (const Tile &t : tiles) n += std::max(1, (t.n + len - 1) / len);
+            const int ns = (longest + len - 1) / len;
+            if (n > per || ns > SK_MAX_SPLIT) break;
+            const double cost = len + 3 + 0.1 * ns;
+            if (cost < best_c) {
+                best_c = cost;
+                best = len;
+            }
         }
-        if (ok && (int)bins.size() <= n_wg) break;
+        for (int t = 0; t < n_tiles; t++) {
+            const int ns = std::max(1, (tiles[t].n + best - 1) / best);
+            const int len = std::max(1, (tiles[t].n + ns - 1) / ns);
+            for (int first = 0; first == 0 || first < tiles[t].n; first += len)
+                bins.push_back({{t, first, std::min(len, tiles[t].n - first)}});
+        }
+    } else {
+        for (double cap = std::max(1.0, (double)total / per);; cap *= 1.02) {
+            bins.assign(1, {});
+            double room = cap;
+            bool ok = true;
+            for (int t = 0; t < n_tiles && ok; t++) {
+                int first = 0, made = 0;
+                do {
+                    if (room < overhead + 1 && !bins.back().empty()) {
+                        bins.push_back({});
+                        room = cap;
+                    }
+                    const int take = std::min(tiles[t].n - first, std::max(1, (int)(room - overhead)));
+                    bins.back().push_back({t, first, take});
+                    first += take;
+                    room -= take + overhead;
+                    if (++made > SK_MAX_SPLIT) ok = false;
+                } while (first < tiles[t].n);
+            }
+            if (ok && (int)bins.size() <= per) break;
+        }
     }
     /* items in slot order: a tile's pieces contiguous, in key order */
-    std::vector<std::vector<int>> pieces_of(tiles.size());
-    std::vector<std::pair<int, int>> where; /* (bin, index in bin) of each piece, by piece id */
-    std::vector<Piece> all;
-    for (int bi = 0; bi < (int)bins.size(); bi++)
-        for (int k = 0; k < (int)bins[bi].size(); k++) {
-            pieces_of[bins[bi][k].tile].push_back((int)all.size());
-            all.push_back(bins[bi][k]);
-            where.push_back({bi, k});
-        }
-    std::vector<int> slot(all.size());
+    struct Placed { int first, count, list; };
+    std::vector<std::vector<Placed>> of(tiles.size());
+    for (int w = 0; w < (int)bins.size(); w++)
+        for (const Piece &pc : bins[w]) of[pc.tile].push_back({pc.first, pc.count, w});
+    lists.assign(bins.size(), {});
     pl.items.clear();
     for (int t = 0; t < (int)tiles.size(); t++) {
         const Tile &tl = tiles[t];
         const SkBatch &sb = pl.sb[tl.batch];
-        const int ns = (int)pieces_of[t].size();
+        std::sort(of[t].begin(), of[t].end(), [](const Placed &a, const Placed &b) { return a.first < b.first; });
+        const int ns = (int)of[t].size();
         for (int sp = 0; sp < ns; sp++) {
-            const Piece &pc = all[pieces_of[t][sp]];
-            slot[pieces_of[t][sp]] = (int)pl.items.size();
+            const Placed &pc = of[t][sp];
             const int kb = tl.lo + pc.first * SMOL_SLAB;
             const int ke = sp == ns - 1 ? tl.hi : tl.lo + (pc.first + pc.count) * SMOL_SLAB;
+            lists[pc.list].push_back((int)pl.items.size());
             pl.items.push_back({tl.batch, tl.row0, kb, std::max(kb, ke), t, ns, sp, sb.fresh_row0 - sb.fresh_pos0});
         }
     }
     pl.n_groups = (int)tiles.size();
-    lists.assign(bins.size(), {});
-    for (int p = 0; p < (int)all.size(); p++) lists[where[p].first].push_back(slot[p]);
+    return two;
 }
 
 /* the pre-pass blocks with their batches */
@@ -1258,26 +1300,48 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     const int pk = ctx->opt[SMOL_OPT_PREFILL_KERNEL];
     const bool precise = ctx->opt[SMOL_OPT_QK_FP16] != 1;
     const bool fa = !cs.dec;
-    bool fb = fa && hd <= 128 && pk != 2;
+    bool fb = fa && pk != 2;
     if (fb) {
         long long tiles = 0;
+        bool widened = false; /* cache rows staged as fresh ones (smol_attn_prefill) */
         for (auto &b : pl.sb) {
             if (b.key_lo < b.fresh_pos0) fb = false;
+            widened |= b.slot >= 0 && b.fresh_pos0 < (b.q_pos0 & ~(SMOL_SLAB - 1));
             tiles += (b.n_rows + 63) / 64;
         }
-        if (pk != 1 && tiles * cs.Hkv < ctx->cu_count / 4) fb = false;
+        if (pk != 1 && hd <= 128 && !widened && tiles * cs.Hkv < ctx->cu_count / 4) fb = false;
     }
     int nt = 1, w = 2, rows_per = 64;
     /* k_attn_fb with two key groups (64-row items, each group half of the
-     * keys; the default) or one key group of eight waves (128-row items whose
-     * key ranges may be split over workgroups and merged: each slab is staged
-     * once for 128 rows and five stages fit with precise QK^T, but at C2's
-     * shape the split items' start-up and merges cost more than that saves) */
-    const bool fb_one = fb && ctx->opt[SMOL_OPT_FB_GROUPS] == 1 && ctx->opt[SMOL_OPT_FB_NT] != 2;
+     * keys, nothing to merge outside the workgroup) or one key group of eight
+     * waves (128-row items whose keys may be split over workgroups; at
+     * head_dim 256 always: four waves, 64-row items). Where one key group's
+     * longest list of slabs and eight steps more (writing partials, the merge
+     * launch) are below the two-group items' steps: few long tiles, which
+     * leave workgroups idle. Measured, two groups / one (us): 500 rows on
+     * 2048 keys, 8 kv heads, 49 / 34; 256 on 1024 26.7 / 21; 1000 on 500 34.7
+     * / 35.8; 300 in a window of 512 19 / 22; 1536 on none 36.6 / 45. */
+    std::vector<std::vector<int>> fill_lists;
+    const int fbg = ctx->opt[SMOL_OPT_FB_GROUPS];
+    bool fb_one = fb && (hd > 128 || (fbg != 2 && ctx->opt[SMOL_OPT_FB_NT] != 2));
+    if (fb_one) {
+        rows_per = hd > 128 ? 64 : 128;
+        const double two = plan_fb_one(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count, fill_lists);
+        double one = 0;
+        for (const auto &l : fill_lists) {
+            double slabs = 3.0 * (l.size() - 1);
+            for (int i : l) slabs += (pl.items[i].key_end - pl.items[i].key_begin + SMOL_SLAB - 1) / SMOL_SLAB;
+            one = std::max(one, slabs);
+        }
+        fb_one = hd > 128 || fbg == 1 || one + 8 < two;
+        if (!fb_one) {
+            pl.items.clear();
+            fill_lists.clear();
+        }
+    }
     if (fb_one) {
         nt = 0; /* the launcher's code for one key group */
         w = 2;
-        rows_per = 128;
     } else if (fb) {
         /* 64-row tiles; SMOL_OPT_FB_NT 2: two row tiles per wave (four waves
          * per workgroup instead of eight) */
@@ -1304,9 +1368,7 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
                       ctx->opt[SMOL_OPT_FB_QPREP] != 1 &&
                       pl.pb.size() == 1 && pl.pb[0].q_tok0 == 0 && pl.pb[0].q_row0 == 0 &&
                       (!(cs.rope && cs.rope_q) || (pl.sb.size() == 1 && pl.sb[0].q_pos0 == pl.pb[0].q_pos0));
-    std::vector<std::vector<int>> fill_lists;
-    if (fb_one) plan_fb_fill(pl, cs.Hkv, G, cs.window, ctx->cu_count, fill_lists);
-    else if (fa) plan_items(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count * w, true, fb);
+    if (fa && !fb_one) plan_items(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count * w, true, fb);
 
     /* workspace; precise QK^T (the default) adds the lo parts of the fp16 Q
      * scratch and of the fresh K */
@@ -1327,11 +1389,6 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     if (fa) {
         if ((rc = dev_reserve(ctx->part_o, std::max<size_t>(1, n_items) * cs.Hkv * rows_per * hd * 4, ctx->stream))) return rc;
         if ((rc = dev_reserve(ctx->part_ml, std::max<size_t>(1, n_items) * cs.Hkv * rows_per * 2 * 4, ctx->stream))) return rc;
-        /* one counter per 256-byte line: the workgroups of different groups count in
-         * at about the same time, and atomics on one line are serialised */
-        if ((rc = dev_reserve(ctx->counters, (size_t)std::max(1, pl.n_groups) * cs.Hkv * 4 * SK_COUNTER_STRIDE,
-                              ctx->stream, true)))
-            return rc;
     }
 
     /* k_attn_fb with more tiles than compute units: one workgroup per unit
@@ -1341,8 +1398,8 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     std::vector<FbItem> fbi;
     int fb_wg = std::max(1, ctx->cu_count / cs.Hkv);
     if (!((int)n_items > fb_wg && ctx->opt[SMOL_OPT_FB_LISTS] != -1)) fb_wg = 0;
-    if (fb_one && ctx->opt[SMOL_OPT_FB_LISTS] != -1) {
-        /* one key group: the planner's filled lists, one workgroup each */
+    if (fb_one) {
+        /* one key group: the planner's lists, one workgroup each */
         fb_wg = (int)fill_lists.size();
         fbi = fb_items(pl, fb_wg, true, &fill_lists);
     } else if (fb) {
@@ -1363,11 +1420,21 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     const size_t o_pblk = 0;
     const size_t o_it = al(o_pblk + pbr.size() * sizeof(PrepBlockB));
     const size_t o_sc = al(o_it + itr.size() * sizeof(SkItemB));
-    const size_t total = al(o_sc + fbi.size() * sizeof(FbItem));
+    std::vector<SkMerge> mrg; /* the split tiles */
+    if (fa)
+        for (size_t i = 0; i < n_items; i += pl.items[i].n_split) {
+            const SkItem &it = pl.items[i];
+            const SkBatch &b = pl.sb[it.batch];
+            if (it.n_split > 1)
+                mrg.push_back({(int)i, it.n_split, it.row0, std::min(rows_per, b.n_rows - it.row0), b.out_tok0});
+        }
+    const size_t o_mg = al(o_sc + fbi.size() * sizeof(FbItem));
+    const size_t total = al(o_mg + mrg.size() * sizeof(SkMerge));
     std::vector<unsigned char> host(total);
     memcpy(host.data() + o_pblk, pbr.data(), pbr.size() * sizeof(PrepBlockB));
     if (!itr.empty()) memcpy(host.data() + o_it, itr.data(), itr.size() * sizeof(SkItemB));
     if (!fbi.empty()) memcpy(host.data() + o_sc, fbi.data(), fbi.size() * sizeof(FbItem));
+    if (!mrg.empty()) memcpy(host.data() + o_mg, mrg.data(), mrg.size() * sizeof(SkMerge));
     if ((rc = upload_desc(ctx, host.data(), total))) return rc;
     unsigned char *dd = (unsigned char *)ctx->desc.p;
 
@@ -1444,7 +1511,6 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     sp.items = (const SkItemB *)(dd + o_it);
     sp.part_o = (float *)ctx->part_o.p;
     sp.part_ml = (float *)ctx->part_ml.p;
-    sp.counters = (int *)ctx->counters.p;
     if (fb) {
         sp.fb_items = (const FbItem *)(dd + o_sc);
         sp.n_wg = fb_wg;
@@ -1461,6 +1527,12 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     if (rc)
         return fail(rc == -1 ? SMOL_ATTN_ERR_UNSUPPORTED : SMOL_ATTN_ERR_DEVICE,
                     "attention launch (hd %d): %s", hd, hipGetErrorString(hipGetLastError()));
+    if (!mrg.empty()) {
+        mk = timing_begin(ctx, 1);
+        if (smol_launch_sk_merge(&sp, (const SkMerge *)(dd + o_mg), (int)mrg.size(), rows_per, hd, ctx->stream,
+                                 mark_a(ctx, mk), mark_b(ctx, mk)))
+            return fail(SMOL_ATTN_ERR_DEVICE, "k_sk_merge: %s", hipGetErrorString(hipGetLastError()));
+    }
     return SMOL_ATTN_OK;
 }
 
@@ -1534,12 +1606,23 @@ extern "C" int smol_attn_prefill_qknorm(smol_attn_ctx *ctx, smol_kv_cache *kv, i
     if ((rc = check_rope(ctx, rope, kv->hd, pos0 + seq_q))) return rc;
     const int Hkv = kv->n_kv, G = n_heads / Hkv, hd = kv->hd;
     Plan pl;
-    const int f0 = pos0 & ~(SMOL_SLAB - 1);
+    /* More than 128 rows (head_dim 256: any): the pre-pass also stages the
+     * cache rows that the call can see, widened to fp16, and k_attn_fb reads
+     * every key from there. That costs 16 + 24 bytes a key element pair
+     * (8000 keys of 8 heads: 11 us); k_attn_fb's slab step, staged by
+     * transfers, is more than twice as fast as k_attn_fa's (attention and
+     * pre-pass, k_attn_fa / widened: 64 tokens of 2 heads a kv head on 8000
+     * keys 41 / 43 us, 128 on 8000 55 / 49, 256 on 4096 57 / 43, 500 on 2048
+     * 60 / 44; head_dim 256, 100 tokens on 1000 38 / 31). The staging stays
+     * below 6 bytes x 32768 keys x n_kv x head_dim. */
+    const int pk = ctx->opt[SMOL_OPT_PREFILL_KERNEL];
+    const bool widen = seq_q * G > 64 && pk != 2 && (pk == 1 || hd > 128 || seq_q * G > 128) && pos0 <= 32768;
+    const int f0 = (widen ? (window > 0 ? std::max(0, pos0 - window + 1) : 0) : pos0) & ~(SMOL_SLAB - 1);
     const int nf = ((pos0 + seq_q + SMOL_SLAB - 1) & ~(SMOL_SLAB - 1)) - f0;
     pl.pb.push_back({0, seq_q, 0, pos0, 0, seq_q, pos0, f0, nf, 0, slot, 0});
     add_q_blocks(pl, 0, seq_q); /* the Q blocks (the longer ones) dispatched first */
     add_fresh_blocks(pl, 0, nf);
-    pl.sb.push_back({seq_q * G, 0, 0, pos0, 0, pos0 + seq_q, 1, f0, 0, slot, 0, 0});
+    pl.sb.push_back({seq_q * G, 0, 0, pos0, widen ? f0 : 0, pos0 + seq_q, 1, f0, 0, slot, 0, 0});
     pl.q_rows = seq_q * G;
     pl.fresh_rows = nf;
     /* short chunks stream the cache like a decode step; long ones are MFMA-bound */

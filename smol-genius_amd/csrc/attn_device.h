@@ -330,30 +330,8 @@ __device__ __forceinline__ uint4 bload(rsrc_t r, unsigned voff, unsigned soff) {
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-/* Device-coherent (SC1) buffer accesses for the split-K partials. The L2s
- * of the XCDs are not coherent with each other; SC1 stores write through to
- * the device coherence point and SC1 loads read from it, so partials pass
- * between workgroups on different XCDs without an L2 write-back or
- * invalidate (what an agent-scope release / acquire fence would cost). */
+/* device-coherent accesses (k_dec's flags): past the XCD's own L2 */
 #define CPOL_SC1 16
-__device__ __forceinline__ void store_f4_sc1(rsrc_t r, unsigned voff, f4 v) {
-    __builtin_amdgcn_raw_buffer_store_b128(u4v{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
-                                               __float_as_uint(v[3])},
-                                           r, voff, 0, CPOL_SC1);
-}
-__device__ __forceinline__ f4 load_f4_sc1(rsrc_t r, unsigned voff) {
-    const u4v v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, CPOL_SC1);
-    return f4{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
-}
-__device__ __forceinline__ void store_f2_sc1(rsrc_t r, unsigned voff, float a, float b) {
-    typedef unsigned u2v __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(u2v{__float_as_uint(a), __float_as_uint(b)}, r, voff, 0, CPOL_SC1);
-}
-__device__ __forceinline__ float2 load_f2_sc1(rsrc_t r, unsigned voff) {
-    typedef unsigned u2v __attribute__((ext_vector_type(2)));
-    const u2v v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, CPOL_SC1);
-    return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
-}
 
 /* One 1 KB direct-to-LDS transfer: lane l's 16 bytes land at lds + 16 l.
  * The LDS address travels in M0. GFX9-family parts (gfx950 included) need

@@ -1,14 +1,15 @@
 /*
  * attn_fb.hip - k_attn_fb: prefill and windowed bidirectional attention over
- * keys that all sit in the fresh fp16 staging.
+ * keys that all sit in the fresh fp16 staging (a call's own keys and, staged
+ * by the same pre-pass, the cache rows it can see).
  */
-#include "attn_splitk.h"
+#include "attn_device.h"
 
 /* ---------------------------------------------------------------- k_attn_fb */
 
 /*
  * Prefill and windowed bidirectional attention over keys that all sit in the
- * fresh fp16 buffers (no cache slabs), for head_dim <= 128. One workgroup
+ * fresh fp16 buffers. One workgroup
  * owns one 64-row tile and needs no other workgroup: its waves form two
  * groups, the groups take the first and second half of the tile's key slabs,
  * and the two partial softmax states are merged through LDS at the end.
@@ -41,20 +42,24 @@
  * PREC (precise QK^T): a stage holds the K image twice, fp16 hi then fp16 lo
  * (the same layout), then V^T; with two key groups the larger stage leaves
  * room for three stages per group instead of five. ONE: a single key group
- * of eight waves (128-row items), which keeps five stages either way. */
+ * of eight waves (128-row items), which keeps five stages either way. At
+ * head_dim 256 there is only ONE, with four waves (64-row items, one wave per
+ * SIMD: a wave's O, Q and the double-buffered fragments take 490 registers)
+ * and three stages of 48 KB (1024 rows in a window of 512, 4 kv heads: 52.8 us
+ * in k_attn_fa, 28.5 here with the merge). */
 template <int HD, int WPG, bool PREC, bool ONE>
 struct FbGeom {
     static constexpr int KS = (HD + 31) / 32;
     static constexpr int DT = (HD + 15) / 16;
     static constexpr int HDP = KS * 32;
-    static constexpr int KROW = 256;
+    static constexpr int KROW = HD <= 128 ? 256 : 512;
     static constexpr int K_BYTES = SMOL_SLAB * KROW;
     static constexpr int KPARTS = PREC ? 2 : 1;
     static constexpr int V_BYTES = 16 * DT * 64;
     static constexpr int STAGE = (KPARTS * K_BYTES + V_BYTES + 1024 * WPG - 1) / (1024 * WPG) * (1024 * WPG);
     static constexpr int NDMA = STAGE / (1024 * WPG); /* DMA instructions per wave per slab */
     static constexpr int GROUPS = ONE ? 1 : 2;
-    static constexpr int NSTG = PREC && !ONE ? 3 : (GROUPS * 5 * STAGE <= 160 * 1024 ? 5 : 4);
+    static constexpr int NSTG = HD > 128 || (PREC && !ONE) ? 3 : (GROUPS * 5 * STAGE <= 160 * 1024 ? 5 : 4);
     static constexpr int GROUP_BYTES = NSTG * STAGE;
 };
 
@@ -64,28 +69,6 @@ struct FbGeom {
  * halves the LDS reads per flop. One MFMA pipe per SIMD is kept busy by a
  * single wave (measured: 16x16x32 f16 MFMAs with independent accumulators
  * issue at the same rate from one wave per SIMD as from two). */
-/* The merge of a split item's group by its last workgroup (merge_group of
- * k_attn_fa on the item's fields), not inlined: its registers then do not add
- * to those of the slab loop, which runs at two waves per SIMD. */
-template <int HD, int ROWS, int TPB>
-__device__ __attribute__((noinline)) void fb_merge(float *part_o, float *part_ml, int *counters, float *out, int Hkv,
-                                                   int Hq, int G, FbItem it, int g, int tid, float *s_o) {
-    /* the fields merge_group reads (passed by value: the kernel's own
-     * argument block stays private to it, so its fields stay uniform) */
-    SkParams p;
-    memset(&p, 0, sizeof(p));
-    p.part_o = part_o; p.part_ml = part_ml; p.counters = counters; p.out = out;
-    p.Hkv = Hkv; p.Hq = Hq; p.G = G;
-    SkItem si;
-    si.batch = 0; si.row0 = it.row0; si.key_begin = it.key_begin; si.key_end = it.key_end;
-    si.group = it.group; si.n_split = it.n_split; si.split = it.split; si.fresh_off = it.fresh_off;
-    SkBatch sb;
-    sb.n_rows = it.n_rows; sb.q_row0 = it.q_row0; sb.out_tok0 = it.out_tok0; sb.q_pos0 = it.q_pos0;
-    sb.key_lo = it.key_lo; sb.key_hi = it.key_hi; sb.causal = it.causal;
-    sb.fresh_pos0 = 0; sb.fresh_row0 = 0; sb.slot = -1; sb.pad0 = sb.pad1 = 0;
-    merge_group<HD, ROWS, 16, TPB>(p, si, sb, it.part, g, tid, s_o);
-}
-
 /* The Q fragments of one 16-row tile straight from the inputs (SkParams.q_in):
  * lane (c, j) holds elements d = 32 ks + 8 j + i of its row (Q scratch row
  * `row` = token * G + head in group, at RoPE position `pos`), so the NeoX
@@ -178,10 +161,10 @@ __device__ __forceinline__ void q_from_input(const SkParams &p, int row, int pos
  * slab is transferred once for all of them), and an item may cover part of
  * its tile's keys (see FbItem), merged across workgroups */
 template <int HD, int NT, bool CAP, bool PREC, bool ONE, bool QIN = false>
-__global__ __launch_bounds__(NT == 1 ? 512 : 256)
-__attribute__((amdgpu_waves_per_eu(NT == 1 ? 2 : 1, NT == 1 ? 2 : 1))) void k_attn_fb(SkParams p) {
-    static_assert(!ONE || NT == 1, "one key group: eight waves of one row tile each");
-    constexpr int WPG = ONE ? 8 : 4 / NT;
+__global__ __launch_bounds__(NT == 1 && HD <= 128 ? 512 : 256)
+__attribute__((amdgpu_waves_per_eu(NT == 1 && HD <= 128 ? 2 : 1, NT == 1 && HD <= 128 ? 2 : 1))) void k_attn_fb(SkParams p) {
+    static_assert(!ONE || NT == 1, "one key group: eight waves of one row tile each (head_dim 256: four)");
+    constexpr int WPG = ONE ? (HD <= 128 ? 8 : 4) : 4 / NT;
     using Gm = FbGeom<HD, WPG, PREC, ONE>;
     constexpr int KS = Gm::KS, DT = Gm::DT, HDP = Gm::HDP, KROW = Gm::KROW;
     constexpr int K_BYTES = Gm::K_BYTES, STAGE = Gm::STAGE, NDMA = Gm::NDMA, NSTG = Gm::NSTG;
@@ -189,11 +172,10 @@ __attribute__((amdgpu_waves_per_eu(NT == 1 ? 2 : 1, NT == 1 ? 2 : 1))) void k_at
     /* one barrier a step and one-step transfers (three stages) */
     constexpr bool B1 = NSTG == 3;
     constexpr int ROWS = 16 * NT * WPG; /* rows of an item */
-    static_assert(HD <= 128, "k_attn_fb covers head_dim <= 128");
+    static_assert(HD <= 128 || ONE, "head_dim 256: one key group");
     static_assert(Gm::GROUPS * Gm::GROUP_BYTES <= 160 * 1024, "LDS");
     static_assert(NSTG >= 3, "the step pipeline keeps three slabs resident");
     static_assert(!PREC || K_BYTES % (1024 * WPG) == 0, "each DMA instruction of a wave lands in one part");
-    static_assert(!ONE || (2 * SK_MERGE_MAX + 2 * ROWS) * 4 <= Gm::GROUP_BYTES, "merge scratch");
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = ONE ? 0 : wave / WPG, wg = wave % WPG;
@@ -201,7 +183,6 @@ __attribute__((amdgpu_waves_per_eu(NT == 1 ? 2 : 1, NT == 1 ? 2 : 1))) void k_at
     const int g = (int)(blockIdx.x % (unsigned)p.Hkv);
     const int w = (int)(blockIdx.x / (unsigned)p.Hkv);
     __shared__ __attribute__((aligned(1024))) unsigned char smem[Gm::GROUPS * Gm::GROUP_BYTES];
-    __shared__ int s_last;
     /* item w, then the rest of this workgroup's list (the host's
      * longest-first assignment when the items outnumber the compute units,
      * where a second wave of workgroups would pay its start-up again) */
@@ -245,7 +226,8 @@ __attribute__((amdgpu_waves_per_eu(NT == 1 ? 2 : 1, NT == 1 ? 2 : 1))) void k_at
         d_part[e] = q * 1024 < K_BYTES ? 0 : q * 1024 < kparts_bytes ? 1 : 2;
         if (d_part[e] < 2) {
             const int qk = d_part[e] == 0 ? q : q - K_BYTES / 1024;
-            const int kr = qk * 4 + (lane >> 4), slot = lane & 15;
+            constexpr int CPR = KROW / 16; /* chunks of a K row's image */
+            const int kr = qk * (64 / CPR) + lane / CPR, slot = lane % CPR;
             const int cb = slot ^ ((kr & 3) | (((kr >> 3) & 3) << 2));
             d_off[e] = cb < HD / 8 ? (unsigned)((kr * HD + cb * 8) * 2) : OOB_OFF;
         } else {
@@ -631,36 +613,22 @@ __attribute__((amdgpu_waves_per_eu(NT == 1 ? 2 : 1, NT == 1 ? 2 : 1))) void k_at
                 }
             }
         } else {
-            /* a split item: publish the unnormalised rows and (m, l) into
-             * slot `part` with device-coherent stores, count in once, and the
-             * group's last workgroup merges (as k_attn_fa's split items) */
+            /* a split item: the unnormalised rows and (m, l) into slot
+             * `part`; k_sk_merge, the next launch, merges the tile's */
             const long long pbase = ((long long)it.part * p.Hkv + g) * ROWS;
-            const rsrc_t ro = make_rsrc(p.part_o + pbase * HD, (long long)ROWS * HD * 4);
-            const rsrc_t rml = make_rsrc(p.part_ml + pbase * 2, (long long)ROWS * 2 * 4);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
+                if (!valid[nt]) continue;
                 const int rr = (wg * NT + nt) * 16 + c;
+                float *po = p.part_o + (pbase + rr) * HD;
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++) {
                     const int d = 16 * dt + 4 * j;
                     if (HD % 16 != 0 && d >= HD) continue;
-                    store_f4_sc1(ro, (unsigned)((rr * HD + d) * 4), o[nt][dt]);
+                    *reinterpret_cast<f4 *>(po + d) = o[nt][dt];
                 }
-                if (j == 0) store_f2_sc1(rml, (unsigned)(rr * 8), m[nt], l[nt]);
+                if (j == 0) *reinterpret_cast<float2 *>(p.part_ml + 2 * (pbase + rr)) = make_float2(m[nt], l[nt]);
             }
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            __builtin_amdgcn_s_waitcnt(0);
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            __syncthreads(); /* every wave's stores are acknowledged (and every stage read is done) */
-            if (tid == 0) {
-                const int prev = __hip_atomic_fetch_add(p.counters + ((long long)it.group * p.Hkv + g) * SK_COUNTER_STRIDE,
-                                                        1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_last = prev == it.n_split - 1;
-            }
-            __syncthreads();
-            if (s_last)
-                fb_merge<HD, ROWS, 64 * WPG>(p.part_o, p.part_ml, p.counters, p.out, p.Hkv, p.Hq, p.G, it, g, tid,
-                                             reinterpret_cast<float *>(smem));
         }
         if (next < 0) break;
         item = next;
@@ -746,6 +714,21 @@ static int launch_fb_qin(const SkParams *sp, dim3 grid, int nt, hipStream_t st, 
     return -1;
 }
 
+/* head_dim 256: one key group of four waves (nt 0) */
+static int launch_fb_256(const SkParams *sp, int n_items, int nt, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    const dim3 grid((sp->n_wg > 0 ? sp->n_wg : n_items) * sp->Hkv), block(256);
+    if (nt != 0 || sp->q_in || (sp->qs_lo && !sp->kf_lo)) return -1;
+    const bool cap = sp->cap2 > 0.0f;
+    if (sp->qs_lo) {
+        if (cap) hipExtLaunchKernelGGL((k_attn_fb<256, 1, true, true, true>), grid, block, 0, st, e0, e1, 0, *sp);
+        else hipExtLaunchKernelGGL((k_attn_fb<256, 1, false, true, true>), grid, block, 0, st, e0, e1, 0, *sp);
+    } else {
+        if (cap) hipExtLaunchKernelGGL((k_attn_fb<256, 1, true, false, true>), grid, block, 0, st, e0, e1, 0, *sp);
+        else hipExtLaunchKernelGGL((k_attn_fb<256, 1, false, false, true>), grid, block, 0, st, e0, e1, 0, *sp);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
 /* precise QK^T (fp16 hi + lo operands) when the Q scratch has its lo part
  * (or Q comes from the inputs) */
 template <int HD>
@@ -765,8 +748,7 @@ static int launch_fb_hd(const SkParams *sp, int n_items, int nt, hipStream_t st,
 
 /* k_attn_fb: every key in the fresh buffers; nt: 1 or 2 row tiles per wave
  * over 64-row items (512 threads for nt 1, 256 for nt 2), or 0: 128-row items
- * of one key group (512 threads; split items merge through part_o / part_ml
- * and the counters); sp->n_wg workgroups per kv head (0: one per item) each
+ * of one key group (512 threads; split items leave partials for k_sk_merge); sp->n_wg workgroups per kv head (0: one per item) each
  * run their list of items; e0 / e1 (may be null): events recorded around the
  * kernel alone */
 extern "C" int smol_launch_fb(const SkParams *sp, int hd, int n_items, int nt, hipStream_t st, hipEvent_t e0,
@@ -778,6 +760,7 @@ extern "C" int smol_launch_fb(const SkParams *sp, int hd, int n_items, int nt, h
     case 80: return launch_fb_hd<80>(sp, n_items, nt, st, e0, e1);
     case 96: return launch_fb_hd<96>(sp, n_items, nt, st, e0, e1);
     case 128: return launch_fb_hd<128>(sp, n_items, nt, st, e0, e1);
+    case 256: return launch_fb_256(sp, n_items, nt, st, e0, e1);
     default: return -1;
     }
 }

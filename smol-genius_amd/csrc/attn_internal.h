@@ -26,8 +26,7 @@
 #include <stdint.h>
 
 #define SMOL_SLAB 32          /* keys per inner step of the attention kernels */
-#define SK_MERGE_MAX 4096     /* max rows * n_split of one split-K merge group (the merge's LDS) */
-#define SK_COUNTER_STRIDE 64  /* ints between two merge groups' counters: one 256-byte line each */
+#define SK_MAX_SPLIT 64       /* items of one split-K merge group at most */
 #define SMOL_ROWS_PER_TILE 16 /* query rows per MFMA tile (16x16x32 f16) */
 
 enum { SMOL_IN_F32 = 0, SMOL_IN_BF16 = 1 };
@@ -74,13 +73,19 @@ typedef struct {
  * [key_begin, key_end), all in the fresh buffers. next: the next item of the
  * same workgroup, or -1. With one key group a tile's keys may be split over
  * several items (a merge group): the item writes its partial into slot
- * `part` and the last of the group to finish merges them. */
+ * `part` and k_sk_merge merges them. */
 typedef struct {
     int key_begin, key_end, fresh_off, row0;
     int n_rows, q_row0, out_tok0, q_pos0;
     int key_lo, key_hi, causal, next;
     int group, n_split, split, part;
 } FbItem;
+
+/* A row tile whose keys were split over several items (k_sk_merge): its
+ * partials sit in the slots first .. first + n_split - 1 */
+typedef struct {
+    int first, n_split, row0, n_rows, out_tok0;
+} SkMerge;
 
 /* Q-scratch format written by k_prep (fresh K / V^T are fp16 in both):
  *   SMOL_STAGE_F16    fp16 (the fp16-MFMA kernels k_attn_fb and k_attn_fa),
@@ -108,7 +113,6 @@ typedef struct {
     const SkItemB *items;      /* k_attn_dec / k_attn_fa items with their batches */
     float *part_o;             /* [item][kv][rows][hd] unnormalised partial outputs */
     float *part_ml;            /* [item][kv][rows][2] (max, sum) */
-    int *counters;             /* [group][kv] at a stride of SK_COUNTER_STRIDE; zero between calls */
     /* k_attn_fb: its items; workgroup w (per kv head) starts at item w and
      * follows the items' next links */
     const FbItem *fb_items;

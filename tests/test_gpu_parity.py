@@ -474,12 +474,50 @@ def test_decode_direct_cache_rows(ctx, sa, oracle, wo, hq, hkv, hd, rt, bf):
 def test_fb_one_key_group(ctx, sa, oracle, case, qk_fp16, opts):
     """k_attn_fb with one key group of eight waves (SMOL_OPT_FB_GROUPS 1):
     128-row items whose long key ranges are split over workgroups and merged
-    by the last of each group. The same cases as the tile lists, with both
+    by k_sk_merge. The same cases as the tile lists, with both
     QK^T modes; with lists and with one workgroup per item the merges add the
     same partials in the same order, so the two launches agree bit for bit."""
     opts(sa.OPT_FB_GROUPS, 1)
     opts(sa.OPT_QK_FP16, qk_fp16)
     test_fb_tile_lists(ctx, sa, oracle, case, opts)
+
+
+@pytest.mark.parametrize("hq,hkv,hd", [(16, 8, 128), (8, 1, 256), (8, 4, 256), (6, 2, 64), (4, 2, 72), (9, 3, 96)])
+def test_prefill_staged_prefix(ctx, sa, oracle, wo, opts, hq, hkv, hd):
+    """A prompt behind a cache prefix through k_attn_fb over the widened
+    prefix (chosen by shape, and forced with one and two key groups) and
+    through k_attn_fa, which reads the cache itself: prefixes that end inside
+    a slab, at one and one past it, windows that start inside the prefix, the
+    softcap, row counts around a tile. Against the oracle without a window,
+    and against k_attn_fa with one: both form the same hi + lo products, so
+    the difference is their fp32 sums' order, about 2^-24 sqrt(slabs) < 1e-5
+    relative."""
+    from smol_genius_amd.workloads import Prefill
+    for P, S, bf, window, cap in [(31, 65, True, 0, 0.0), (32, 64, False, 0, 0.0), (333, 129, False, 0, 0.0),
+                                  (1000, 40, True, 0, 0.0), (1, 200, True, 0, 0.0), (700, 150, False, 65, 0.0),
+                                  (700, 97, True, 300, 30.0), (95, 130, False, 1, 0.0)]:
+        print("staged prefix", hq, hkv, hd, P, S, bf, window, cap, flush=True)
+        wl = Prefill("t", hq, hkv, hd, P, S, 1e5, seed=700 + P + S, in_bf16=bf)
+        x = wl.inputs()
+        outs = {}
+        for name, kernel, groups in (("auto", 0, 0), ("one", 1, 1), ("two", 1, 2), ("fa", 2, 0)):
+            opts(sa.OPT_PREFILL_KERNEL, kernel)
+            opts(sa.OPT_FB_GROUPS, groups)
+            kv = sa.KVCache(ctx, 1, 1, hkv, hd, P + S)
+            kv.write(0, 0, 0, x["cache_k"], x["cache_v"])
+            rope = sa.RopeTable(ctx, hd, wl.theta, 0)
+            outs[name] = sa.prefill(ctx, kv, 0, 0, rope, P, dev(x["q"], bf), dev(x["k"], bf), dev(x["v"], bf), hq,
+                                    wl.scale, window=window, cap=cap).cpu().numpy()
+            k_rows, v_rows = kv.read(0, 0, 0, P)  # the prefix is only read
+            np.testing.assert_array_equal(k_rows, x["cache_k"])
+            np.testing.assert_array_equal(v_rows, x["cache_v"])
+        opts(sa.OPT_PREFILL_KERNEL, 0)
+        opts(sa.OPT_FB_GROUPS, 0)
+        fa = outs.pop("fa").astype(np.float64)
+        for name, got in outs.items():
+            if not window and not cap:
+                assert_parity(got, wo.prefill(oracle, wl, x), "staged prefix %s P=%d S=%d" % (name, P, S))
+            assert np.linalg.norm(got - fa) <= 1e-5 * np.linalg.norm(fa), (name, P, S, window, cap)
 
 
 @pytest.mark.parametrize("window,cap", [(16, 0.0), (0, 2.0), (1, 0.0), (40, 1.5), (1, 3.0)])
