@@ -190,10 +190,13 @@ struct smol_attn_ctx {
     DevBuf qs32; /* fp32 Q scratch of the decode kernel */
     DevBuf out32; /* fp32 result of a call whose output is bf16 */
     DevBuf dec_part; /* k_dec partial slots and flags */
-    /* device flags, 256 bytes: word 0 is set by kernels when fp16 staging
-     * overflows, word 32 (its own 128-byte line) by a k_dec merger that gave
-     * up waiting for its splits; synchronize reads and clears both */
+    /* flags, 256 bytes of pinned host memory that kernels write to (only when
+     * there is something to report) and the host reads without a copy: word 0
+     * is set when fp16 staging overflows, word 32 (its own 128-byte line) by
+     * a k_dec merger that gave up waiting for its splits; synchronize reads
+     * and clears both */
     int *range_flag = nullptr;
+    hipEvent_t mark = nullptr; /* smol_internal_mark */
     /* kernel arguments of k_dec and k_attn_win, built in place per context
      * (several KB: kept off the stack; one thread per context, so no two
      * calls build them at once) */
@@ -367,12 +370,14 @@ extern "C" int smol_attn_ctx_create(int device, void *stream, smol_attn_ctx **ou
     int rc = scratch_setup(device);
     if (!rc) rc = check_xcd_dispatch(c);
     if (!rc) {
-        if (hipMalloc((void **)&c->range_flag, 256) != hipSuccess ||
-            hipMemset(c->range_flag, 0, 256) != hipSuccess)
+        if (hipHostMalloc((void **)&c->range_flag, 4 * SMOL_FLAG_WORDS,
+                          hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) == hipSuccess)
+            memset(c->range_flag, 0, 4 * SMOL_FLAG_WORDS);
+        else
             rc = fail(SMOL_ATTN_ERR_NOMEM, "range flag: %s", hipGetErrorString(hipGetLastError()));
     }
     if (rc) {
-        if (c->range_flag) hipFree(c->range_flag);
+        if (c->range_flag) hipHostFree(c->range_flag);
         delete c;
         return rc;
     }
@@ -388,7 +393,8 @@ extern "C" int smol_attn_ctx_destroy(smol_attn_ctx *ctx) {
                       &ctx->qs32, &ctx->out32, &ctx->dec_part};
     for (DevBuf *b : bufs)
         if (b->p) hipFree(b->p);
-    if (ctx->range_flag) hipFree(ctx->range_flag);
+    if (ctx->range_flag) hipHostFree(ctx->range_flag);
+    if (ctx->mark) hipEventDestroy(ctx->mark);
     for (auto &s : ctx->ring) {
         if (s.h) hipHostFree(s.h);
         if (s.ev) hipEventDestroy(s.ev);
@@ -403,16 +409,13 @@ extern "C" int smol_attn_ctx_destroy(smol_attn_ctx *ctx) {
     return SMOL_ATTN_OK;
 }
 
-extern "C" int smol_attn_ctx_synchronize(smol_attn_ctx *ctx) {
-    if (!ctx) return fail(SMOL_ATTN_ERR_ARG, "ctx is NULL");
-    HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+/* the error that the finished kernels flagged, if any; clears the flags */
+static int take_flags(smol_attn_ctx *ctx) {
+    volatile int *f = ctx->range_flag;
     int flag[SMOL_FLAG_WORDS] = {};
-    HIP_TRY(hipMemcpy(flag, ctx->range_flag, sizeof(flag), hipMemcpyDeviceToHost));
-    if (flag[0] || flag[SMOL_FLAG_MERGE]) {
-        const int zero[SMOL_FLAG_WORDS] = {};
-        HIP_TRY(hipMemcpy(ctx->range_flag, zero, sizeof(zero), hipMemcpyHostToDevice));
-    }
+    flag[0] = f[0];
+    flag[SMOL_FLAG_MERGE] = f[SMOL_FLAG_MERGE];
+    f[0] = f[SMOL_FLAG_MERGE] = 0;
     if (flag[SMOL_FLAG_MERGE])
         return fail(SMOL_ATTN_ERR_TIMEOUT, "a decode split-K merge gave up waiting for its splits (the affected "
                     "rows are NaN)");
@@ -420,6 +423,28 @@ extern "C" int smol_attn_ctx_synchronize(smol_attn_ctx *ctx) {
         return fail(SMOL_ATTN_ERR_RANGE, "a staged Q, K or V value was not finite or reached 65520 in magnitude "
                     "(fp16 staging of the prefill and bidirectional kernels)");
     return SMOL_ATTN_OK;
+}
+
+extern "C" int smol_attn_ctx_synchronize(smol_attn_ctx *ctx) {
+    if (!ctx) return fail(SMOL_ATTN_ERR_ARG, "ctx is NULL");
+    HIP_TRY(hipSetDevice(ctx->device));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return take_flags(ctx);
+}
+
+/* for qkn_attn.hip: what smol_attn_ctx_synchronize would report of the work
+ * enqueued before the mark, without waiting for what follows it (which must
+ * not raise flags itself) */
+extern "C" int smol_internal_mark(smol_attn_ctx *ctx) {
+    if (!ctx->mark) HIP_TRY(hipEventCreateWithFlags(&ctx->mark, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(ctx->mark, ctx->stream));
+    return SMOL_ATTN_OK;
+}
+extern "C" int smol_internal_check_mark(smol_attn_ctx *ctx) {
+    HIP_TRY(hipEventSynchronize(ctx->mark));
+    const int rc = take_flags(ctx);
+    if (rc) hipStreamSynchronize(ctx->stream); /* an error leaves nothing running, as synchronize does */
+    return rc;
 }
 
 extern "C" void *smol_attn_ctx_stream(smol_attn_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }

@@ -498,17 +498,17 @@ __device__ __forceinline__ float block_sum256(float v, float *red) {
 }
 
 /* One workgroup per row s of [seq][dim] bf16 arrays:
- *   p non-NULL:     q = w_post ? nrm(p, w_post) : p;  x = add(x, q)  (x updated)
- *   w_next non-NULL: xn = nrm(x, w_next)               (of the updated x)
+ *   p non-NULL:     q = w_post ? nrm(p, w_post) : p;  xo = add(x, q)  (xo may be x)
+ *   w_next non-NULL: xn = nrm(xo, w_next)   (p NULL: of x)
  * (the Gemma 3 post-sublayer norm, the residual add and the next sublayer's
  * input norm, qkn_bf16_decoder.c:551-557 and 567-570, in one pass). xn may
  * equal x only when p is NULL; each thread reads back only the elements it
  * wrote itself. */
-__global__ __launch_bounds__(256) void k_bf16_rows(uint16_t *x, const uint16_t *p, const float *w_post,
+__global__ __launch_bounds__(256) void k_bf16_rows(const uint16_t *x, uint16_t *xo, const uint16_t *p, const float *w_post,
                                                    const float *w_next, uint16_t *xn, int dim, float eps) {
     __shared__ float red[4];
     const long long base = (long long)blockIdx.x * dim;
-    uint16_t *xr = x + base;
+    const uint16_t *xr = x + base;
     float ss = 0.0f;
     if (p) {
         const uint16_t *pr = p + base;
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256) void k_bf16_rows(uint16_t *x, const uint16_t *
             float q = bfw(pr[i]);
             if (w_post) q = bfw(bftr((q * rp) * w_post[i]));
             const uint16_t xb = bftr(bfw(xr[i]) + q);
-            xr[i] = xb;
+            xo[base + i] = xb;
             const float v = bfw(xb);
             ss = fmaf(v, v, ss);
         }
@@ -538,7 +538,8 @@ __global__ __launch_bounds__(256) void k_bf16_rows(uint16_t *x, const uint16_t *
     if (!w_next) return;
     const float r = 1.0f / sqrtf(block_sum256(ss, red) / (float)dim + eps);
     uint16_t *nr = xn + base;
-    for (int i = threadIdx.x; i < dim; i += 256) nr[i] = bftr((bfw(xr[i]) * r) * w_next[i]);
+    const uint16_t *xs = p ? xo + base : xr;
+    for (int i = threadIdx.x; i < dim; i += 256) nr[i] = bftr((bfw(xs[i]) * r) * w_next[i]);
 }
 
 /* out[i] = geglu(bf(gu[2i]), bf(gu[2i + 1])) over n = seq * inter outputs
@@ -1065,6 +1066,18 @@ extern "C" int smol_rms_norm_dev(smol_attn_ctx *ctx, float *out, const float *x,
     return 0;
 }
 
+/* smol_bf16_add_norm_dev with the sum written to xo (x itself, or an array
+ * that overlaps none of the others) */
+extern "C" int smol_internal_bf16_add_norm(smol_attn_ctx *ctx, const uint16_t *x, uint16_t *xo, const uint16_t *p,
+                                           const float *p_norm, const float *next_norm, uint16_t *xn, int seq, int dim,
+                                           float eps) {
+    LHIP(hipSetDevice(smol_internal_ctx_device(ctx)));
+    hipStream_t st = static_cast<hipStream_t>(smol_attn_ctx_stream(ctx));
+    hipLaunchKernelGGL(k_bf16_rows, dim3((unsigned)seq), dim3(256), 0, st, x, xo, p, p_norm, next_norm, xn, dim, eps);
+    LHIP(hipGetLastError());
+    return 0;
+}
+
 extern "C" int smol_bf16_add_norm_dev(smol_attn_ctx *ctx, uint16_t *x, const uint16_t *p, const float *p_norm,
                                       const float *next_norm, uint16_t *xn, int seq, int dim, float eps) {
     if (!ctx) return lfail(SMOL_ATTN_ERR_ARG, "smol_bf16_add_norm_dev: null context");
@@ -1077,11 +1090,7 @@ extern "C" int smol_bf16_add_norm_dev(smol_attn_ctx *ctx, uint16_t *x, const uin
     };
     if (overlap(x, p) || (p && overlap(xn, x)) || overlap(xn, p) || (xn && xn != x && overlap(xn, x)))
         return lfail(SMOL_ATTN_ERR_ARG, "smol_bf16_add_norm_dev: overlapping arrays (xn may equal x only without p)");
-    LHIP(hipSetDevice(smol_internal_ctx_device(ctx)));
-    hipStream_t st = static_cast<hipStream_t>(smol_attn_ctx_stream(ctx));
-    hipLaunchKernelGGL(k_bf16_rows, dim3((unsigned)seq), dim3(256), 0, st, x, p, p_norm, next_norm, xn, dim, eps);
-    LHIP(hipGetLastError());
-    return 0;
+    return smol_internal_bf16_add_norm(ctx, x, x, p, p_norm, next_norm, xn, seq, dim, eps);
 }
 
 extern "C" int smol_bf16_rms_norm_dev(smol_attn_ctx *ctx, uint16_t *out, const uint16_t *x, const float *weight,
@@ -1095,8 +1104,8 @@ extern "C" int smol_bf16_rms_norm_dev(smol_attn_ctx *ctx, uint16_t *out, const u
         return lfail(SMOL_ATTN_ERR_ARG, "smol_bf16_rms_norm_dev: out partly overlaps x");
     LHIP(hipSetDevice(smol_internal_ctx_device(ctx)));
     hipStream_t st = static_cast<hipStream_t>(smol_attn_ctx_stream(ctx));
-    /* the kernel reads x through its residual pointer and writes xn; nothing is added */
-    hipLaunchKernelGGL(k_bf16_rows, dim3((unsigned)seq), dim3(256), 0, st, const_cast<uint16_t *>(x),
+    /* nothing is added */
+    hipLaunchKernelGGL(k_bf16_rows, dim3((unsigned)seq), dim3(256), 0, st, x, (uint16_t *)nullptr,
                        (const uint16_t *)nullptr, (const float *)nullptr, weight, out, dim, eps);
     LHIP(hipGetLastError());
     return 0;

@@ -290,3 +290,56 @@ def test_step_graph(sa, oracle, dorc, name, cfg, dim, inter, act, gemma, sliding
             graph.close()
         for b in blks:
             b.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("rows", [3, 40])
+@pytest.mark.parametrize("gemma", [False, True], ids=["qwen3", "gemma3"])
+def test_layer_range_error_leaves_x(sa, bf16, rows, gemma):
+    """A V row beyond the fp16 staging's range: the prefill layer raises
+    SmolAttnRangeError, x keeps its bits (the output projection and gate_up
+    have run beside the check by then), and the next call is not affected."""
+    dim, inter, H, Hkv, hd = 256, 384, 4, 2, 64
+    owner = ctypes.create_string_buffer(256)
+    blk = sa.QknAttn(owner, n_layers=1, n_heads=H, n_kv_heads=Hkv, head_dim=hd, eps=1e-6, rope_theta=1e6,
+                     rope_local_theta=0.0, rope_type=0, sliding_window=0, attn_logit_softcap=0.0,
+                     bf16=1 if bf16 else 0, on_device=1, device=0, max_seq=64)
+
+    def d(a):
+        if a is None:
+            return None
+        a = np.ascontiguousarray(a)
+        return torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).cuda()
+
+    def layer(big):
+        wv = synth.normal(903, (Hkv * hd, dim), 1.0 / np.sqrt(dim))
+        if big:
+            wv[5] *= 1e6
+        w = dict(input_norm=_norm_w(900, dim), wq=_proj(901, H * hd, dim), wk=_proj(902, Hkv * hd, dim),
+                 wv=synth.f32_to_bf16_bits(wv), wo=_proj(904, dim, H * hd), post_attn_norm=_norm_w(905, dim),
+                 pre_ffn_norm=_norm_w(906, dim) if gemma else None, post_ffn_norm=_norm_w(907, dim) if gemma else None,
+                 gate_up=_proj(908, 2 * inter, dim), down=_proj(909, dim, inter))
+        return sa.QknLayerWeights(**{k: d(v) for k, v in w.items()})
+
+    def call(xd, w):
+        if bf16:
+            blk.layer_prefill_bf16(0, 0, xd, w, dim, inter)
+        else:
+            blk.layer_prefill(0, 0, xd, w, dim, inter, 1)
+        blk.synchronize()
+        return xd.cpu()
+
+    try:
+        blk.set_layer(0, 0, None, None)
+        x = synth.normal(910, (rows, dim))
+        x = d(synth.f32_to_bf16_bits(x)) if bf16 else d(x)
+        good, bad = layer(False), layer(True)
+        print("range error", bf16, rows, gemma, flush=True)
+        want = call(x.clone(), good)
+        y = x.clone()
+        with pytest.raises(sa.SmolAttnRangeError):
+            call(y, bad)
+        assert torch.equal(y.cpu(), x.cpu())
+        assert torch.equal(call(y, good), want) and not torch.equal(want, x.cpu())
+    finally:
+        blk.close()
