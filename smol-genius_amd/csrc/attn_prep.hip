@@ -347,54 +347,78 @@ __device__ __forceinline__ float sqrt_rn(float x) {
  *   x0' = trunc(fma(x0, c, -(x1 * s))), x1' = trunc(fma(x1, c, x0 * s))
  * with c, s the table entries of column 2i. hd is a multiple of 8. */
 /* rows [0, seq H) of x (weight w) and then rows [0, seq H2) of x2 (weight
- * w2; x2 NULL: none), one thread per head row */
+ * w2; x2 NULL: none), NORM_ROPE_ROWS head rows a workgroup: the rows go
+ * through LDS (loads and stores whole rows at a time), one thread per row
+ * forms its r, then all of them take the 16-byte chunks in turn. With one
+ * thread doing a whole row from memory, 256 rows a workgroup, 333 tokens of
+ * 24 heads at head_dim 128 ran on 32 workgroups, each thread a chain of
+ * strided loads: 11.9 us; now 4.7. LDS: rows of hd bf16 and 16 bytes (eight
+ * lanes reading one chunk of eight rows hit distinct banks). */
+#define NORM_ROPE_ROWS 32
 __global__ __launch_bounds__(256) void k_bf16_norm_rope(uint16_t *x, const float *w, uint16_t *x2, const float *w2,
                                                         float eps, const float *cos_t, const float *sin_t, int pos0,
                                                         int seq, int H, int H2, int hd) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_nr[];
+    __shared__ float s_ri[NORM_ROPE_ROWS];
+    const int tid = threadIdx.x;
     const long long rows1 = (long long)seq * H, rows = rows1 + (x2 ? (long long)seq * H2 : 0);
-    const long long step = (long long)gridDim.x * blockDim.x;
-    for (long long rr = (long long)blockIdx.x * blockDim.x + threadIdx.x; rr < rows; rr += step) {
-        const bool second = rr >= rows1;
-        const long long r = second ? rr - rows1 : rr;
-        const int Hr = second ? H2 : H;
-        const float *w_r = second ? w2 : w;
-        uint4 *row = reinterpret_cast<uint4 *>((second ? x2 : x) + r * hd);
-        const int n8 = hd >> 3;
+    const long long rr0 = (long long)blockIdx.x * NORM_ROPE_ROWS;
+    const int n = (int)(rows - rr0 < NORM_ROPE_ROWS ? rows - rr0 : NORM_ROPE_ROWS);
+    const int n8 = hd >> 3, stride = hd * 2 + 16;
+    auto chunk = [&](int r, int c8) __attribute__((always_inline)) {
+        return reinterpret_cast<uint4 *>(lds_nr + r * stride + c8 * 16);
+    };
+    auto row_at = [&](int r) __attribute__((always_inline)) {
+        const long long rr = rr0 + r;
+        return reinterpret_cast<uint4 *>(rr >= rows1 ? x2 + (rr - rows1) * hd : x + rr * hd);
+    };
+    for (int e = tid; e < n * n8; e += 256) {
+        const int r = e / n8, c8 = e - r * n8;
+        *chunk(r, c8) = row_at(r)[c8];
+    }
+    __syncthreads();
+    if (tid < n) {
         float ri = 1.0f;
-        if (w_r) {
+        if (rr0 + tid >= rows1 ? w2 : w) {
             float ss = 0.0f;
             for (int c8 = 0; c8 < n8; c8++) {
                 float v[8];
-                unpack_bf16x8(row[c8], v);
+                unpack_bf16x8(*chunk(tid, c8), v);
 #pragma unroll
                 for (int i = 0; i < 8; i++) ss = __fmaf_rn(v[i], v[i], ss);
             }
             ri = __fdiv_rn(1.0f, sqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)hd), eps)));
         }
-        const float *ct = cos_t ? cos_t + (long long)(pos0 + r / Hr) * hd : nullptr;
-        const float *st = cos_t ? sin_t + (long long)(pos0 + r / Hr) * hd : nullptr;
-        for (int c8 = 0; c8 < n8; c8++) {
-            float v[8];
-            unpack_bf16x8(row[c8], v);
-            if (w_r) {
+        s_ri[tid] = ri;
+    }
+    __syncthreads();
+    for (int e = tid; e < n * n8; e += 256) {
+        const int r = e / n8, c8 = e - r * n8;
+        const bool second = rr0 + r >= rows1;
+        const float *w_r = second ? w2 : w;
+        float v[8];
+        unpack_bf16x8(*chunk(r, c8), v);
+        if (w_r) {
+            const float ri = s_ri[r];
 #pragma unroll
-                for (int i = 0; i < 8; i++) v[i] = __uint_as_float(__float_as_uint(__fmul_rn(__fmul_rn(v[i], ri), w_r[c8 * 8 + i])) & 0xFFFF0000u);
-            }
-            if (ct) {
-#pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    const float c = ct[c8 * 8 + i], s = st[c8 * 8 + i];
-                    const float x0 = v[i], x1 = v[i + 1];
-                    v[i] = __fmaf_rn(x0, c, -__fmul_rn(x1, s));
-                    v[i + 1] = __fmaf_rn(x1, c, __fmul_rn(x0, s));
-                }
-            }
-            uint32_t o[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                o[k] = (__float_as_uint(v[2 * k]) >> 16) | (__float_as_uint(v[2 * k + 1]) & 0xFFFF0000u);
-            row[c8] = make_uint4(o[0], o[1], o[2], o[3]);
+            for (int i = 0; i < 8; i++) v[i] = __uint_as_float(__float_as_uint(__fmul_rn(__fmul_rn(v[i], ri), w_r[c8 * 8 + i])) & 0xFFFF0000u);
         }
+        if (cos_t) {
+            const long long t = pos0 + (second ? (rr0 + r - rows1) / H2 : (rr0 + r) / H);
+            const float *ct = cos_t + t * hd + c8 * 8, *st = sin_t + t * hd + c8 * 8;
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                const float c = ct[i], s = st[i];
+                const float x0 = v[i], x1 = v[i + 1];
+                v[i] = __fmaf_rn(x0, c, -__fmul_rn(x1, s));
+                v[i + 1] = __fmaf_rn(x1, c, __fmul_rn(x0, s));
+            }
+        }
+        uint32_t o[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            o[k] = (__float_as_uint(v[2 * k]) >> 16) | (__float_as_uint(v[2 * k + 1]) & 0xFFFF0000u);
+        row_at(r)[c8] = make_uint4(o[0], o[1], o[2], o[3]);
     }
 }
 
@@ -480,9 +504,9 @@ extern "C" int smol_launch_bf16_norm_rope(uint16_t *x, const float *w, uint16_t 
                            x2 ? H2 : 0, hd);
         return hipGetLastError() == hipSuccess ? 0 : -3;
     }
-    const int blocks = (int)std::min<long long>((rows + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_bf16_norm_rope, dim3(blocks), dim3(256), 0, st, x, w, x2, w2, eps, cos_t, sin_t, pos0, seq,
-                       H, H2, hd);
+    const unsigned blocks = (unsigned)((rows + NORM_ROPE_ROWS - 1) / NORM_ROPE_ROWS);
+    hipLaunchKernelGGL(k_bf16_norm_rope, dim3(blocks), dim3(256), NORM_ROPE_ROWS * ((size_t)hd * 2 + 16), st, x, w, x2,
+                       w2, eps, cos_t, sin_t, pos0, seq, H, H2, hd);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -91,8 +91,19 @@ __device__ __forceinline__ void split_frag(const float *v, b8 &hi, b8 &lo) {
     lo = as_b8(make_uint4(lw[0], lw[1], lw[2], lw[3]));
 }
 
+/* v truncated to bf16, and the bf16 decoder's GeGLU of a truncated (gate, up)
+ * pair before its own truncation: every step rounded as written
+ * (qkn_bf16_decoder.c:235-251) */
+__device__ __forceinline__ float bf16_trunc(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+__device__ __forceinline__ float bf16_geglu(float g, float u) {
+    const float x3 = __fmul_rn(__fmul_rn(g, g), g);
+    const float inner = __fmul_rn(0.7978845608028654f, __fadd_rn(g, __fmul_rn(0.044715f, x3)));
+    return __fmul_rn(__fmul_rn(__fmul_rn(0.5f, g), __fadd_rn(1.0f, tanhf(inner))), u);
+}
+
 /* Outputs n .. n + 3 (n < NN, a multiple of 4) of row m from their sums v:
- * row scale r (NORM), bias, activation, residual, store */
+ * row scale r (NORM), bias, activation, residual, store (a bf16 y truncates;
+ * its activation is the bf16 decoder's GeGLU) */
 template <bool YBF, bool NORM>
 __device__ __forceinline__ void gemm_store4(const GemmParams &p, void *Yt, int m, int n, int NN, float (&v)[4],
                                             float r) {
@@ -105,7 +116,12 @@ __device__ __forceinline__ void gemm_store4(const GemmParams &p, void *Yt, int m
     }
     if (has_act) {
         const int col = n / 2;
-        float o[2] = {act_fn(v[0], p.act) * v[1], act_fn(v[2], p.act) * v[3]};
+        float o[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            if constexpr (YBF) o[e] = bf16_geglu(bf16_trunc(v[2 * e]), bf16_trunc(v[2 * e + 1]));
+            else o[e] = act_fn(v[2 * e], p.act) * v[2 * e + 1];
+        }
         const long long yi = (long long)m * ycols + col;
         const int nv = min(2, ycols - col);
         if (p.res) {

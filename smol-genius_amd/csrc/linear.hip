@@ -897,6 +897,23 @@ extern "C" int smol_internal_linear_bf16_ops(smol_attn_ctx *ctx, uint16_t *y, co
     return run_gemv(ctx, st, x, x_f32_trunc == 0, true, seq, in_dim, 1, &sg, nullptr, &bo);
 }
 
+/* The bf16 decoder's gate_up projection and GeGLU for more rows than a GEMV
+ * takes, in one k_gemm launch: the (gate, up) pairs are truncated and joined at
+ * the tile's end, with the bits of smol_linear_dev and smol_bf16_geglu_dev
+ * (333 rows, 3072 pairs: k_bf16_geglu's 5 us and 6 MB of traffic less).
+ * Returns 1, launching nothing, where k_gemm cannot take the operands. */
+extern "C" int smol_internal_linear_bf16_geglu(smol_attn_ctx *ctx, uint16_t *g, const uint16_t *x, const uint16_t *w,
+                                               int seq, int in_dim, int out_dim) {
+    if (seq <= SMOL_LINEAR_GEMV_MAX_SEQ || in_dim <= 0 || in_dim % 8 != 0 || (out_dim & 1) || !aligned16(x) ||
+        !aligned16(w) || (long long)out_dim * in_dim * 2 > 0x7FFF0000LL || (long long)seq * in_dim > INT_MAX / 4 ||
+        (long long)seq * in_dim * 4 > 0x7FFF0000LL || (long long)seq * out_dim > INT_MAX / 4)
+        return 1;
+    LHIP(hipSetDevice(smol_internal_ctx_device(ctx)));
+    const GemvFuse f{nullptr, 0.0f, SMOL_LINEAR_ACT_GEGLU, nullptr};
+    return run_gemm(ctx, static_cast<hipStream_t>(smol_attn_ctx_stream(ctx)), g, true, x, true, w, nullptr, seq, in_dim,
+                    out_dim, &f);
+}
+
 extern "C" int smol_linear_qkv_dev(smol_attn_ctx *ctx, void *q, void *k, void *v, int y_dtype, const void *x,
                                    int x_dtype, const uint16_t *wq, const uint16_t *wk, const uint16_t *wv, int seq,
                                    int in_dim, int q_dim, int kv_dim) {

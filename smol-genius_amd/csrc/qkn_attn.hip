@@ -27,6 +27,8 @@
 
 extern "C" int smol_internal_fail(int code, const char *msg);
 extern "C" int smol_internal_mark(smol_attn_ctx *ctx);
+extern "C" int smol_internal_linear_bf16_geglu(smol_attn_ctx *ctx, uint16_t *g, const uint16_t *x, const uint16_t *w,
+                                               int seq, int in_dim, int out_dim);
 extern "C" int smol_internal_check_mark(smol_attn_ctx *ctx);
 extern "C" int smol_internal_bf16_add_norm(smol_attn_ctx *ctx, const uint16_t *x, uint16_t *xo, const uint16_t *p,
                                            const float *p_norm, const float *next_norm, uint16_t *xn, int seq, int dim,
@@ -380,8 +382,12 @@ int run_layer_bf16(Binding *b, int layer, int pos, int n, uint16_t *x, const smo
                                                 nullptr)))
             return rc;
     } else {
-        if ((rc = smol_linear_dev(ctx, gu, BF, xn, BF, w->gate_up, nullptr, n, dim, 2 * inter))) return rc;
-        if ((rc = smol_bf16_geglu_dev(ctx, g, gu, n, inter))) return rc;
+        rc = smol_internal_linear_bf16_geglu(ctx, g, xn, w->gate_up, n, dim, 2 * inter);
+        if (rc < 0) return rc;
+        if (rc == 1) {
+            if ((rc = smol_linear_dev(ctx, gu, BF, xn, BF, w->gate_up, nullptr, n, dim, 2 * inter))) return rc;
+            if ((rc = smol_bf16_geglu_dev(ctx, g, gu, n, inter))) return rc;
+        }
     }
     if (!decode && (rc = smol_internal_check_mark(ctx))) return rc;
     if (few && !w->post_ffn_norm)
