@@ -301,6 +301,7 @@ void k_gemm(const GemmParams p) {
 
 /* ------------------------------------------------------------------ launch */
 
+extern "C" int smol_launch_gemm_rs(const GemmParams *p, bool ybf, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 extern "C" int smol_launch_gemm_kw(const GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
                                    hipEvent_t e1);
 
@@ -321,10 +322,7 @@ static int launch_gemm_t(const GemmParams &p, bool norm, hipStream_t st, hipEven
  * with an fp32 x each wave should own rows of its own (WN = 1), so each
  * element is split once per workgroup (two waves across the outputs both
  * split the same fragment: the split, not the matrix cores, bounds the fp32
- * steps); the 192-row tile keeps two waves across the outputs, since its
- * eight waves' rows would not be whole 16-row tiles otherwise, and eight
- * waves (two per SIMD, one hiding the other's LDS and split latency) beat
- * four with rows of their own */
+ * steps); the 192-row tile with an fp32 x is k_gemm_rs (gemm_rs.hip) */
 template <int BM, int BN, int WNF, int WMF, int WNB, int WMB>
 static int launch_gemm_b(const GemmParams &p, bool xbf, bool ybf, bool norm, hipStream_t st, hipEvent_t e0,
                          hipEvent_t e1) {
@@ -385,7 +383,10 @@ extern "C" int smol_launch_gemm(GemmParams *p, int cfg, bool xbf, bool ybf, hipS
     if (cfg > 2) return smol_launch_gemm_kw(p, cfg, xbf, ybf, st, e0, e1);
     const bool norm = p->g != nullptr;
     switch (cfg) {
-    case 0: return launch_gemm_b<192, 192, 2, 4, 2, 4>(*p, xbf, ybf, norm, st, e0, e1);
+    case 0:
+        if (!xbf) return smol_launch_gemm_rs(p, ybf, st, e0, e1);
+        return ybf ? launch_gemm_t<192, 192, 2, 4, true, true>(*p, false, st, e0, e1)
+                   : launch_gemm_t<192, 192, 2, 4, true, false>(*p, false, st, e0, e1);
     case 1: return launch_gemm_b<128, 128, 1, 8, 2, 4>(*p, xbf, ybf, norm, st, e0, e1);
     default: return launch_gemm_b<64, 64, 1, 4, 2, 2>(*p, xbf, ybf, norm, st, e0, e1);
     }

@@ -749,7 +749,7 @@ int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, int seg_align = 
         float f32[4], bf16[4];
     };
     static const Cost cost[GEMM_CFGS] = {
-        {1, 64, {0.00f, 9.66f, 26.07f, 0.523f}, {0.00f, 6.63f, 14.06f, 0.003f}},
+        {1, 64, {0.00f, 10.14f, 24.32f, 0.311f}, {0.00f, 6.63f, 14.06f, 0.003f}},
         {1, 64, {0.00f, 6.21f, 13.45f, 0.257f}, {0.00f, 5.07f, 9.75f, 0.00f}},
         {2, 64, {0.00f, 4.69f, 7.37f, 0.121f}, {0.00f, 2.82f, 6.94f, 0.049f}},
         {1, 256, {0.00f, 6.35f, 4.40f, 0.075f}, {1.50f, 3.71f, 3.42f, 0.035f}},

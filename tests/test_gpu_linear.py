@@ -296,6 +296,29 @@ def test_gemm_k_over_waves(ctx, sa, oracle, tile):
         ctx.set_option(sa.OPT_GEMM_TILE, 0)
 
 
+@pytest.mark.parametrize("n_in", [8, 64, 72, 128, 200, 320])
+def test_gemm_register_staged(ctx, sa, oracle, n_in):
+    """k_gemm_rs (fp32 x, 192 x 192 tiles, forced) with one K step and less,
+    two, and a remainder: stages ahead of K's end are zeros; rows and outputs
+    one past a tile and one short of it."""
+    ctx.set_option(sa.OPT_GEMM_TILE, 1)
+    try:
+        for seq, n_out, norm in [(193, 191, False), (191, 194, True)]:
+            print("gemm rs", seq, n_in, n_out, norm, flush=True)
+            x, w, b = linear_inputs(8900 + n_in + n_out, seq, n_in, n_out, True)
+            if norm:
+                g = (1.0 + 0.1 * synth.normal(8901, (n_in,))).astype(np.float32)
+                y = sa.linear_ops(ctx, dev(x), dev_bits(w), dev(b), norm_weight=dev(g), eps=1e-6)
+                ctx.synchronize()
+                assert_parity(y.cpu().numpy(), oracle.linear_bf16(oracle.rms_norm(x, g, 1e-6), w, b), "gemm rs norm")
+            else:
+                y = sa.linear(ctx, dev(x), dev_bits(w), dev(b))
+                ctx.synchronize()
+                check(y.cpu().numpy(), oracle.linear_bf16(x, w, b), x, w, b, "gemm rs %d" % n_in)
+    finally:
+        ctx.set_option(sa.OPT_GEMM_TILE, 0)
+
+
 def test_gemm_full_prefill_shapes(ctx, sa, oracle):
     """Qwen3-0.6B projections of a 1536-token prefill: sampled rows against the
     oracle, every row against a float64 product on the device."""
