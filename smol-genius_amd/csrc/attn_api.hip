@@ -6,7 +6,7 @@
  * and keys each kernel block covers), copies them to the device through a
  * ring of pinned buffers, and enqueues two kernels on the context's stream:
  * k_prep (RoPE + cache append + staging) and one attention kernel:
- * k_attn_fb (prefill over new keys), k_attn_fa (prefill over a cache prefix)
+ * k_attn_fb (prefill), k_attn_fa (prefill of few rows)
  * or k_attn_dec (decode and short chunks). Nothing here computes attention on
  * the host; without a GPU every entry point fails with SMOL_ATTN_ERR_NO_GPU.
  */
@@ -1007,7 +1007,7 @@ struct DecCall {
  * another to finish before it starts. Workgroup b is slot b / n_xcc of XCD
  * b % n_xcc; slots past an XCD's list are idle. SMOL_OPT_DEC_SLABS > 0
  * instead cuts every unit into workgroups of that many slabs. */
-static void plan_decode(smol_attn_ctx *ctx, const DecCall &dc, int Hkv, int window, int n_rb, int fit, int min_per,
+static void plan_decode(smol_attn_ctx *ctx, const DecCall &dc, int hd, int Hkv, int window, int n_rb, int fit, int min_per,
                         std::vector<DecItem> &items) {
     const int nx = ctx->n_xcc;
     const int n_seq = (int)dc.seqs.size();
@@ -1049,7 +1049,14 @@ static void plan_decode(smol_attn_ctx *ctx, const DecCall &dc, int Hkv, int wind
             const double per = std::max<double>(min_per, (double)work * n_rb / fit);
             long long used = 0;
             for (Unit *u : mine) {
-                const int cap = std::min(DEC_MAX_SPLIT, std::max(1, u->ns));
+                /* a short decode unit stays whole: publishing, polling and
+                 * merging cost more than a few slabs a wave (us a layer, one
+                 * workgroup / split: head_dim 128, 200 keys 9.6 / 11.2, 330
+                 * 10.6 / 11.5, 400 11.9 / 11.8, 700 13.9 / 11.8; head_dim 64,
+                 * 520 keys 9.1 / 10.3, 700 9.9 / 10.0, 1000 11.1 / 10.3; at
+                 * 256 min_per keeps the same line) */
+                const bool whole = dc.direct && (long long)u->ns * hd <= 12 * 128;
+                const int cap = whole ? 1 : std::min(DEC_MAX_SPLIT, std::max(1, u->ns));
                 u->n_split = std::max(1, std::min(cap, (int)std::lround(u->ns / per)));
                 used += (long long)u->n_split * n_rb;
             }
@@ -1142,12 +1149,12 @@ static int run_decode(smol_attn_ctx *ctx, const CallShape &cs, const DecCall &dc
      * longer splits win (C4: 23.4 -> 21.5 us) */
     const int min_per = hd > 128 ? 2 * nw : nw;
     std::vector<DecItem> items;
-    plan_decode(ctx, *pdc, cs.Hkv, cs.window, n_rb, fit, min_per, items);
+    plan_decode(ctx, *pdc, hd, cs.Hkv, cs.window, n_rb, fit, min_per, items);
     if (dc.noalloc && items.size() > DEC_ARG_ITEMS && !pdc->whole) {
         whole_dc = dc;
         whole_dc.whole = true;
         pdc = &whole_dc;
-        plan_decode(ctx, *pdc, cs.Hkv, cs.window, n_rb, fit, min_per, items);
+        plan_decode(ctx, *pdc, hd, cs.Hkv, cs.window, n_rb, fit, min_per, items);
     }
     if (gd && items.size() > DEC_ARG_ITEMS)
         return fail(SMOL_ATTN_ERR_UNSUPPORTED, "captured decode: %d workgroups exceed the kernel arguments' %d",
@@ -1633,8 +1640,8 @@ extern "C" int smol_attn_prefill_qknorm(smol_attn_ctx *ctx, smol_kv_cache *kv, i
     Plan pl;
     /* More than 128 rows (head_dim 256: any): the pre-pass also stages the
      * cache rows that the call can see, widened to fp16, and k_attn_fb reads
-     * every key from there. That costs 16 + 24 bytes a key element pair
-     * (8000 keys of 8 heads: 11 us); k_attn_fb's slab step, staged by
+     * every key from there. That costs 4 bytes read and 6 written per key
+     * and element (8000 keys of 8 heads: 11 us); k_attn_fb's slab step, staged by
      * transfers, is more than twice as fast as k_attn_fa's (attention and
      * pre-pass, k_attn_fa / widened: 64 tokens of 2 heads a kv head on 8000
      * keys 41 / 43 us, 128 on 8000 55 / 49, 256 on 4096 57 / 43, 500 on 2048

@@ -352,7 +352,7 @@ __device__ __forceinline__ float sqrt_rn(float x) {
  * forms its r, then all of them take the 16-byte chunks in turn. With one
  * thread doing a whole row from memory, 256 rows a workgroup, 333 tokens of
  * 24 heads at head_dim 128 ran on 32 workgroups, each thread a chain of
- * strided loads: 11.9 us; now 4.7. LDS: rows of hd bf16 and 16 bytes (eight
+ * strided loads: 11.9 us; now 5.5. LDS: rows of hd bf16 and 16 bytes (eight
  * lanes reading one chunk of eight rows hit distinct banks). */
 #define NORM_ROPE_ROWS 32
 __global__ __launch_bounds__(256) void k_bf16_norm_rope(uint16_t *x, const float *w, uint16_t *x2, const float *w2,
