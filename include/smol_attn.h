@@ -138,10 +138,10 @@ SMOL_ATTN_API int smol_attn_ctx_timing_read(smol_attn_ctx *ctx, double *ms, int 
 #define SMOL_OPT_FB_GROUPS 12     /* k_attn_fb at head_dim <= 128: 0: chosen per call; 1: one key group of
                                    * eight waves over 128-row items (long items' keys split over workgroups
                                    * and merged); 2: two key groups over 64-row items */
-#define SMOL_OPT_GEMM_TILE 13     /* k_gemm (projections of more than 4 rows): 0: tile chosen per shape;
-                                   * 1, 2, 3: 192 x 192, 128 x 128, 64 x 64 (rows x outputs); 4 to 9: K split
-                                   * over the waves of a workgroup, 64 x 64 over eight and over four, 32 x 64
-                                   * over eight, 32 x 32 over four, 16 x 32 and 16 x 16 over eight */
+#define SMOL_OPT_GEMM_TILE 13     /* projections of more than 4 rows: 0: tile chosen per shape; 1 to 8: 192 x 192,
+                                   * 128 x 128, 64 x 64, 64 x 128, 32 x 64, 32 x 32, 16 x 32, 16 x 16 (rows x
+                                   * outputs). A row's results are the same bits in every tile, and so do not
+                                   * depend on how many rows (more than 4) a call has */
 #define SMOL_OPT_FB_QPREP 14      /* k_attn_fb at head_dim 64 / 128 with precise QK^T and no per-head
                                    * Q norm: 0: each item rotates and scales its own Q rows from the
                                    * inputs; 1: the pre-pass stages them (as for k_attn_fa) */

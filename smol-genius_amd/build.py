@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libsmol_attn.so")
-SOURCES = ["attn_prep.hip", "attn_decode.hip", "attn_fa.hip", "attn_fb.hip", "attn_win.hip", "attn_api.hip", "qkn_attn.hip", "linear.hip", "gemm.hip", "gemm_kw.hip", "gemm_rs.hip"]
+SOURCES = ["attn_prep.hip", "attn_decode.hip", "attn_fa.hip", "attn_fb.hip", "attn_win.hip", "attn_api.hip", "qkn_attn.hip", "linear.hip", "gemm.hip", "gemm_sw.hip", "gemm_rs.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("SMOL_ATTN_ARCH", "gfx950")
 

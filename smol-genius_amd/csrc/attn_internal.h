@@ -276,8 +276,8 @@ typedef struct {
     DecItem items[DEC_ARG_ITEMS];
 } DecParams;
 
-/* ---- k_gemm (gemm.hip) and k_gemm_kw (gemm_kw.hip): the projections on bf16 MFMA ---- */
-#define GEMM_CFGS 9 /* tile configurations of both (smol_gemm_tile) */
+/* ---- k_gemm (gemm.hip), k_gemm_rs (gemm_rs.hip) and k_gemm_sw (gemm_sw.hip): the projections on bf16 MFMA ---- */
+#define GEMM_CFGS 8 /* their tile configurations (smol_gemm_tile) */
 struct GemmParams {
     const uint16_t *w; /* [N][K] bf16 */
     const void *x;     /* [M][K] fp32 or bf16 */

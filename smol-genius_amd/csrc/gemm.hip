@@ -22,13 +22,13 @@
  * Tiling. One workgroup computes a BN x BM tile (outputs x rows) with
  * v_mfma_f32_16x16x32_bf16: A = W rows (outputs), B = x rows, so a lane's
  * four accumulator values are four consecutive outputs of one row (one
- * 16-byte store, and both members of a gate / up pair). Three tile sizes
- * (192 x 192 and 128 x 128 with eight waves, 64 x 64 with four and two
- * workgroups per compute unit: two waves per SIMD in each); the host picks
- * one from the launch's rounds over the device. With a bf16 x the waves
- * form a 2 x (NW / 2) grid; with an fp32 x each wave of the two smaller
- * tiles owns rows of its own (1 x NW) and so splits each element once per
- * workgroup. K advances 64 at a time through NSTG LDS
+ * 16-byte store, and both members of a gate / up pair). Here the large tiles,
+ * 192 x 192 (with a bf16 x; k_gemm_rs takes an fp32 one) and 128 x 128, eight
+ * waves, two per SIMD; gemm_sw.hip has the smaller ones. Every tile of the
+ * three kernels forms an output's sum in one order, so the host may pick any
+ * (gemm_cfg, linear.hip) without a change of bits. With a bf16 x the waves
+ * form a 2 x (NW / 2) grid; with an fp32 x each wave owns rows of its own
+ * (1 x NW) and so splits each element once per workgroup. K advances 64 at a time through NSTG LDS
  * stages (three where they fit in 150 KB, else two): W, x and the norm
  * weight all by direct-to-LDS transfers (buffer_load ... lds), the next
  * stages in flight while one is multiplied. LDS rows are 128 or 256 bytes
@@ -72,8 +72,7 @@ __device__ __forceinline__ unsigned swz(int row, int q, int rb) {
 } // namespace
 
 template <int BM, int BN, int WN, int WM, bool XBF, bool YBF, bool NORM>
-__global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(WN * WM * (BM >= 128 ? 1 : 2) / 4,
-                                                                             WN * WM * (BM >= 128 ? 1 : 2) / 4)))
+__global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(WN * WM / 4, WN * WM / 4)))
 void k_gemm(const GemmParams p) {
     using Gm = GemmGeom<BM, BN, XBF, WN, WM>;
     constexpr int NW = Gm::NW;
@@ -302,14 +301,14 @@ void k_gemm(const GemmParams p) {
 /* ------------------------------------------------------------------ launch */
 
 extern "C" int smol_launch_gemm_rs(const GemmParams *p, bool ybf, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
-extern "C" int smol_launch_gemm_kw(const GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
+extern "C" int smol_launch_gemm_sw(const GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
                                    hipEvent_t e1);
 
 template <int BM, int BN, int WN, int WM, bool XBF, bool YBF>
-static int launch_gemm_t(const GemmParams &p, bool norm, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+static int launch_gemm_t(const GemmParams &p, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     const dim3 grid((unsigned)(GEMM_XCD * p.per_xcd)), block(64 * WN * WM);
     if constexpr (!XBF) {
-        if (norm) {
+        if (p.g) {
             hipExtLaunchKernelGGL((k_gemm<BM, BN, WN, WM, false, YBF, true>), grid, block, 0, st, e0, e1, 0, p);
             return hipGetLastError() == hipSuccess ? 0 : -3;
         }
@@ -318,25 +317,10 @@ static int launch_gemm_t(const GemmParams &p, bool norm, hipStream_t st, hipEven
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-/* wave layouts, (WNF x WMF) for an fp32 x and (WNB x WMB) for a bf16 x:
- * with an fp32 x each wave should own rows of its own (WN = 1), so each
- * element is split once per workgroup (two waves across the outputs both
- * split the same fragment: the split, not the matrix cores, bounds the fp32
- * steps); the 192-row tile with an fp32 x is k_gemm_rs (gemm_rs.hip) */
-template <int BM, int BN, int WNF, int WMF, int WNB, int WMB>
-static int launch_gemm_b(const GemmParams &p, bool xbf, bool ybf, bool norm, hipStream_t st, hipEvent_t e0,
-                         hipEvent_t e1) {
-    if (xbf) return ybf ? launch_gemm_t<BM, BN, WNB, WMB, true, true>(p, false, st, e0, e1)
-                        : launch_gemm_t<BM, BN, WNB, WMB, true, false>(p, false, st, e0, e1);
-    return ybf ? launch_gemm_t<BM, BN, WNF, WMF, false, true>(p, norm, st, e0, e1)
-               : launch_gemm_t<BM, BN, WNF, WMF, false, false>(p, norm, st, e0, e1);
-}
-
 /* the configurations the host may choose (rows of x = BM, outputs = BN):
- * 0-2 k_gemm, 3-8 k_gemm_kw (gemm_kw.hip), of which 4 and 6 split K over four
- * waves and the others over eight */
+ * 0 k_gemm, or k_gemm_rs with an fp32 x; 1 k_gemm; 2-7 k_gemm_sw */
 extern "C" int smol_gemm_tile(int cfg, int *bm, int *bn) {
-    static const int t[GEMM_CFGS][2] = {{192, 192}, {128, 128}, {64, 64}, {64, 64}, {64, 64},
+    static const int t[GEMM_CFGS][2] = {{192, 192}, {128, 128}, {64, 64}, {64, 128},
                                         {32, 64},   {32, 32},   {16, 32}, {16, 16}};
     if (cfg < 0 || cfg >= GEMM_CFGS) return -1;
     *bm = t[cfg][0];
@@ -344,50 +328,55 @@ extern "C" int smol_gemm_tile(int cfg, int *bm, int *bn) {
     return 0;
 }
 
-/* p's tile fields are filled here from the configuration; K % 8 == 0 and a
- * 16-byte aligned W and x are the caller's to check */
-extern "C" int smol_launch_gemm(GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
-                                hipEvent_t e1) {
+/* p's tile fields from its M, N, K and the configuration: the region split
+ * with the fewest operand bytes per XCD (x rows of its row blocks + W rows of
+ * its column blocks); a grid smaller than the split in either direction is
+ * dealt contiguously. Returns the tiles of an XCD's list, negative when there
+ * is no such configuration */
+extern "C" int smol_gemm_plan(GemmParams *p, int cfg, bool xbf) {
     int bm, bn;
     if (smol_gemm_tile(cfg, &bm, &bn)) return -1;
-    if (xbf && p->g) return -1;
     p->tiles_m = (p->M + bm - 1) / bm;
     const int tiles_n = (p->N + bn - 1) / bn;
     p->tiles = p->tiles_m * tiles_n;
-    if (p->tiles <= 0) return 0;
-    if (p->rm > 0) {
-        /* the region split with the fewest operand bytes per XCD (x rows
-         * of its row blocks + W rows of its column blocks); a grid smaller
-         * than the split in either direction keeps the contiguous deal */
-        static const int splits[4][2] = {{1, 8}, {2, 4}, {4, 2}, {8, 1}};
-        const double xrow = (double)p->K * (xbf ? 2 : 4), wrow = (double)p->K * 2;
-        double best = 1e300;
-        p->rm = 0;
-        for (const auto &sp : splits) {
-            if (sp[0] > p->tiles_m || sp[1] > tiles_n) continue;
-            const double bytes = (double)((p->tiles_m + sp[0] - 1) / sp[0]) * bm * xrow +
-                                 (double)((tiles_n + sp[1] - 1) / sp[1]) * bn * wrow;
-            if (bytes < best) {
-                best = bytes;
-                p->rm = sp[0];
-                p->rn = sp[1];
-            }
+    static const int splits[4][2] = {{1, 8}, {2, 4}, {4, 2}, {8, 1}};
+    const double xrow = (double)p->K * (xbf ? 2 : 4), wrow = (double)p->K * 2;
+    double best = 1e300;
+    p->rm = 0;
+    for (const auto &sp : splits) {
+        if (sp[0] > p->tiles_m || sp[1] > tiles_n) continue;
+        const double bytes = (double)((p->tiles_m + sp[0] - 1) / sp[0]) * bm * xrow +
+                             (double)((tiles_n + sp[1] - 1) / sp[1]) * bn * wrow;
+        if (bytes < best) {
+            best = bytes;
+            p->rm = sp[0];
+            p->rn = sp[1];
         }
     }
-    if (p->rm > 0) {
-        const int hm = (p->tiles_m + p->rm - 1) / p->rm, hn = (tiles_n + p->rn - 1) / p->rn;
-        p->per_xcd = hm * hn;
-    } else {
+    if (p->rm > 0)
+        p->per_xcd = ((p->tiles_m + p->rm - 1) / p->rm) * ((tiles_n + p->rn - 1) / p->rn);
+    else
         p->per_xcd = (p->tiles + GEMM_XCD - 1) / GEMM_XCD;
-    }
-    if (cfg > 2) return smol_launch_gemm_kw(p, cfg, xbf, ybf, st, e0, e1);
-    const bool norm = p->g != nullptr;
-    switch (cfg) {
-    case 0:
+    return p->per_xcd;
+}
+
+/* K % 8 == 0 and a 16-byte aligned W and x are the caller's to check. Wave
+ * layouts: with an fp32 x each wave should own rows of its own (two waves
+ * across the outputs both split the same fragment: the split, not the matrix
+ * cores, bounds the fp32 steps) */
+extern "C" int smol_launch_gemm(GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
+                                hipEvent_t e1) {
+    if (xbf && p->g) return -1;
+    if (smol_gemm_plan(p, cfg, xbf) < 0) return -1;
+    if (p->tiles <= 0) return 0;
+    if (cfg > 1) return smol_launch_gemm_sw(p, cfg, xbf, ybf, st, e0, e1);
+    if (cfg == 0) {
         if (!xbf) return smol_launch_gemm_rs(p, ybf, st, e0, e1);
-        return ybf ? launch_gemm_t<192, 192, 2, 4, true, true>(*p, false, st, e0, e1)
-                   : launch_gemm_t<192, 192, 2, 4, true, false>(*p, false, st, e0, e1);
-    case 1: return launch_gemm_b<128, 128, 1, 8, 2, 4>(*p, xbf, ybf, norm, st, e0, e1);
-    default: return launch_gemm_b<64, 64, 1, 4, 2, 2>(*p, xbf, ybf, norm, st, e0, e1);
+        return ybf ? launch_gemm_t<192, 192, 2, 4, true, true>(*p, st, e0, e1)
+                   : launch_gemm_t<192, 192, 2, 4, true, false>(*p, st, e0, e1);
     }
+    if (xbf) return ybf ? launch_gemm_t<128, 128, 2, 4, true, true>(*p, st, e0, e1)
+                        : launch_gemm_t<128, 128, 2, 4, true, false>(*p, st, e0, e1);
+    return ybf ? launch_gemm_t<128, 128, 1, 8, false, true>(*p, st, e0, e1)
+               : launch_gemm_t<128, 128, 1, 8, false, false>(*p, st, e0, e1);
 }

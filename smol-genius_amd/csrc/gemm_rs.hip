@@ -7,8 +7,10 @@
  * reaches here. k_gemm holds an fp32 x in LDS as loaded, so both waves that
  * share a fragment read 32 bytes an element pair more and split it again, in
  * the way of their MFMAs. Here the stages come through registers and are split
- * once, on the way into LDS, by the thread that loaded them: 51.2 -> 46.5 us
- * there, 180 -> 154 us for 2048 -> 12288. (The smaller tiles and a bf16 x gain
+ * once, on the way into LDS, by the thread that loaded them: 51.2 -> 47.5 us
+ * there, 180 -> 162 us for 2048 -> 12288. (The norm's squares in eight parts a
+ * row take 46.4 and 159 us, but leave the scale other last bits than the other
+ * tiles' four.) (The smaller tiles and a bf16 x gain
  * nothing: 128 x 128 25.3 / 25.4 us, bf16 192 x 192 37.2 / 39.9; k_gemm's
  * direct transfers stay there. A third LDS stage, with the next step's
  * fragments read during the products, spilled registers: 58 us.)
@@ -99,13 +101,21 @@ void k_gemm_rs(const GemmParams p) {
             float v[8] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w),
                           __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
             if constexpr (NORM) {
+                /* the row's four running sums (chunks lq, then lq + 4: k_gemm's
+                 * order) rest in lanes lq < 4, go to lanes lq + 4 and come back */
+                auto squares = [&](float t) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int b = 0; b < 8; b++) t = fmaf(v[b], v[b], t);
+                    return t;
+                };
+                const float up = __uint_as_float(__builtin_amdgcn_update_dpp(
+                    0, __float_as_uint(squares(ss[e])), 0x114 /* row_shr:4 */, 0xf, 0xf, true));
+                ss[e] = __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(squares(up)),
+                                                                    0x104 /* row_shl:4 */, 0xf, 0xf, true));
                 const uint4 g0 = r.g[0], g1 = r.g[1];
                 const uint32_t g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    ss[e] = fmaf(v[b], v[b], ss[e]);
-                    v[b] *= __uint_as_float(g[b]);
-                }
+                for (int b = 0; b < 8; b++) v[b] *= __uint_as_float(g[b]);
             }
             b8 h, l;
             split_frag(v, h, l);
@@ -167,13 +177,14 @@ void k_gemm_rs(const GemmParams p) {
             __syncthreads();
         }
 
-    /* the rows' scale: threads 8 r .. 8 r + 7 hold row r's partial sums */
+    /* the rows' scale: threads 8 r .. 8 r + 3 hold row r's partial sums, added
+     * as row_sum4 does */
     if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < XL; e++) {
             float t = ss[e];
-#pragma unroll
-            for (int m = 1; m < 8; m <<= 1) t += __shfl_xor(t, m, 64);
+            t += __shfl_xor(t, 2, 64);
+            t += __shfl_xor(t, 1, 64);
             if (lq == 0) s_rinv[lr + TPB / 8 * e] = 1.0f / sqrtf(t / (float)K + p.eps);
         }
         __syncthreads();

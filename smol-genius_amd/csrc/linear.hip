@@ -20,8 +20,8 @@
  *            step is issued before the first FMA. Sums: per-lane fp32, then
  *            a wave all-reduce (cross-row swaps + DPP row rotations), then
  *            the kp waves' totals in a fixed order through LDS.
- *   k_gemm   longer inputs (gemm.hip; gemm_kw.hip for a few to a few
- *            hundred rows): bf16 MFMA tiles with the input
+ *   k_gemm   longer inputs (gemm.hip; gemm_rs.hip for large fp32
+ *            tiles, gemm_sw.hip for small ones): bf16 MFMA tiles with the input
  *            RMSNorm, the bias, the gated activation and the residual add
  *            fused; an fp32 x is split into bf16 hi + lo as it is staged
  *            (y = W x_hi + W x_lo, x carried to ~2^-17 relative, the
@@ -54,6 +54,7 @@ extern "C" int smol_launch_to_bf16_trunc(const float *x, uint16_t *y, long long 
 extern "C" int smol_internal_ctx_cus(smol_attn_ctx *ctx);
 extern "C" int smol_internal_ctx_option(smol_attn_ctx *ctx, int option);
 extern "C" int smol_gemm_tile(int cfg, int *bm, int *bn);
+extern "C" int smol_gemm_plan(GemmParams *p, int cfg, bool xbf);
 extern "C" int smol_launch_gemm(GemmParams *p, int cfg, bool xbf, bool ybf, hipStream_t st, hipEvent_t e0,
                                 hipEvent_t e1);
 
@@ -731,33 +732,28 @@ int run_gemv_rows(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const v
 }
 
 /* The configuration for an M x N product over K (smol_gemm_tile): the one
- * of least estimated time. With R rounds of workgroups over the device (one
- * workgroup per compute unit a round; two of k_gemm's 64 x 64, which are
- * resident together) a launch takes about
+ * of least estimated time. With R rounds of workgroups (the longest XCD's tiles
+ * over its compute units) a launch takes about
  *     a + R (b + c K) + d (weight MB)   us,
- * K in thousands, rounded up to what the waves split it into. The constants
- * are fitted (least squares of the relative error) to the measured times of
- * every configuration at 8 to 1536 rows, 1024 to 12288 outputs and K = 1024
- * to 6144, weights not in L2; there the choice is within 1.5% of the best
- * configuration on average, 33% at worst (700 bf16 rows, 1024 -> 6144), and
- * within 4% of the best k_gemm tile everywhere. Where the lines fall: for
- * K = 1024, N = 1024 k_gemm_kw up to about 700 rows, for N = 6144 up to about
- * 128. */
-int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, int seg_align = 0) {
-    struct Cost {
-        int per_cu, kstep; /* workgroups per compute unit; K of one step of all its waves */
-        float f32[4], bf16[4];
-    };
-    static const Cost cost[GEMM_CFGS] = {
-        {1, 64, {0.00f, 10.14f, 24.32f, 0.311f}, {0.00f, 6.63f, 14.06f, 0.003f}},
-        {1, 64, {0.00f, 6.21f, 13.45f, 0.257f}, {0.00f, 5.07f, 9.75f, 0.00f}},
-        {2, 64, {0.00f, 4.69f, 7.37f, 0.121f}, {0.00f, 2.82f, 6.94f, 0.049f}},
-        {1, 256, {0.00f, 6.35f, 4.40f, 0.075f}, {1.50f, 3.71f, 3.42f, 0.035f}},
-        {1, 128, {3.53f, 2.49f, 5.30f, 0.091f}, {3.42f, 1.26f, 3.44f, 0.024f}},
-        {1, 256, {0.466f, 4.68f, 2.95f, 0.078f}, {2.27f, 2.39f, 2.71f, 0.048f}},
-        {1, 256, {3.85f, 1.22f, 2.11f, 0.085f}, {3.76f, 0.571f, 1.28f, 0.038f}},
-        {1, 512, {1.54f, 3.23f, 1.23f, 0.094f}, {2.72f, 2.12f, 0.850f, 0.066f}},
-        {1, 512, {2.68f, 2.21f, 0.782f, 0.107f}, {3.23f, 1.15f, 0.530f, 0.041f}},
+ * K in thousands. The constants are fitted (least squares of the relative
+ * error) to the measured times of every configuration at 5 to 2048 rows, 640 to
+ * 12288 outputs and K = 640 to 6144, weights not in L2, for a plain fp32 x, one
+ * with the norm and a bf16 x; over those 484 products the choice is within 0.7%
+ * of the best configuration on average, 26% at worst (1300 bf16 rows, 6144 ->
+ * 2048: 83.9 us against 66.6). The bits are the same in every one of them.
+ * Where the lines fall (rows up to which a k_gemm_sw tile is chosen): N = 1024,
+ * K = 1024 to 3072: 2048 and more; N = 6144, K = 1024: 320; N = 12288, K = 2048
+ * with the norm: 128. */
+int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, bool norm, int seg_align = 0) {
+    static const float cost[GEMM_CFGS][3][4] = {
+        {{0.0f, 7.89f, 25.9f, 0.0737f}, {0.0f, 9.66f, 27.5f, 0.186f}, {0.0f, 6.91f, 17.1f, 0.0f}},
+        {{0.0f, 3.59f, 14.9f, 0.137f}, {0.0f, 5.56f, 17.9f, 0.0342f}, {0.0f, 5.43f, 10.5f, 0.0f}},
+        {{4.68f, 0.0f, 5.37f, 0.0745f}, {2.13f, 3.21f, 7.37f, 0.00928f}, {3.83f, 1.26f, 3.52f, 0.00656f}},
+        {{0.0f, 4.63f, 8.72f, 0.0996f}, {0.0f, 6.23f, 10.1f, 0.0325f}, {0.573f, 5.81f, 5.87f, 0.0f}},
+        {{2.05f, 2.25f, 4.12f, 0.0f}, {1.99f, 3.19f, 4.88f, 0.00881f}, {3.73f, 1.04f, 2.65f, 0.0192f}},
+        {{1.84f, 2.19f, 2.91f, 0.0f}, {2.72f, 2.11f, 4.03f, 0.0125f}, {3.77f, 0.865f, 1.62f, 0.0166f}},
+        {{2.26f, 1.75f, 1.86f, 0.00487f}, {2.28f, 2.98f, 2.09f, 0.0f}, {3.46f, 0.716f, 1.07f, 0.0339f}},
+        {{3.32f, 0.963f, 1.29f, 0.0105f}, {2.53f, 2.61f, 1.68f, 0.0104f}, {3.11f, 0.899f, 0.758f, 0.0319f}},
     };
     const int forced = smol_internal_ctx_option(ctx, SMOL_OPT_GEMM_TILE);
     if (forced >= 1 && forced <= GEMM_CFGS) {
@@ -765,20 +761,21 @@ int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, int seg_align = 
         smol_gemm_tile(forced - 1, &bm, &bn);
         return seg_align % bn == 0 ? forced - 1 : -1;
     }
-    const int cus = smol_internal_ctx_cus(ctx);
+    const int per_xcd_cus = std::max(1, smol_internal_ctx_cus(ctx) / 8);
+    const double k = K / 1024.0, mb = (double)N * K * 2e-6;
     int best = -1;
     double best_t = 1e300;
     for (int cfg = 0; cfg < GEMM_CFGS; cfg++) {
         int bm, bn;
         smol_gemm_tile(cfg, &bm, &bn);
         if (seg_align % bn != 0) continue; /* segment boundaries on tile edges */
-        const Cost &q = cost[cfg];
-        const float *f = xbf ? q.bf16 : q.f32;
-        const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const long long slots = (long long)cus * q.per_cu;
-        const double rounds = (double)((tiles + slots - 1) / slots);
-        const double k = (double)((K + q.kstep - 1) / q.kstep) * q.kstep / 1024;
-        const double t = f[0] + rounds * (f[1] + k * f[2]) + f[3] * ((double)N * K * 2e-6);
+        GemmParams p{};
+        p.M = M;
+        p.N = N;
+        p.K = K;
+        const int rounds = (smol_gemm_plan(&p, cfg, xbf) + per_xcd_cus - 1) / per_xcd_cus;
+        const float *f = cost[cfg][xbf ? 2 : norm ? 1 : 0];
+        const double t = f[0] + rounds * (f[1] + k * f[2]) + f[3] * mb;
         if (t < best_t) {
             best_t = t;
             best = cfg;
@@ -809,10 +806,9 @@ int run_gemm(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const void *
     p.M = seq;
     p.N = out;
     p.K = in;
-    p.rm = 1; /* the launcher chooses the region split */
     hipEvent_t e0 = nullptr, e1 = nullptr;
     smol_internal_timing_events(ctx, LIN_TIMING_KIND, &e0, &e1);
-    const int rc = smol_launch_gemm(&p, gemm_cfg(ctx, seq, out, in, xbf), xbf, ybf, st, e0, e1);
+    const int rc = smol_launch_gemm(&p, gemm_cfg(ctx, seq, out, in, xbf, p.g != nullptr), xbf, ybf, st, e0, e1);
     if (rc) return lfail(SMOL_ATTN_ERR_DEVICE, rc == -1 ? "k_gemm: unsupported operands" : "k_gemm launch failed");
     return 0;
 }
@@ -829,7 +825,7 @@ int run_gemm_qkv(smol_attn_ctx *ctx, hipStream_t st, void *q, void *k, void *v, 
         (f && f->norm_w && !aligned16(f->norm_w)) || (long long)q_dim * in * 2 > 0x7FFF0000LL ||
         (long long)kv_dim * in * 2 > 0x7FFF0000LL || (long long)seq * in * 4 > 0x7FFF0000LL)
         return 1;
-    const int cfg = gemm_cfg(ctx, seq, q_dim + 2 * kv_dim, in, xbf, std::gcd(q_dim, kv_dim));
+    const int cfg = gemm_cfg(ctx, seq, q_dim + 2 * kv_dim, in, xbf, f && f->norm_w, std::gcd(q_dim, kv_dim));
     if (cfg < 0) return 1;
     GemmParams p{};
     p.w = wq;
@@ -842,7 +838,6 @@ int run_gemm_qkv(smol_attn_ctx *ctx, hipStream_t st, void *q, void *k, void *v, 
     p.M = seq;
     p.N = q_dim + 2 * kv_dim;
     p.K = in;
-    p.rm = 1;
     p.nseg = 3;
     p.seg_c[0] = 0;
     p.seg_c[1] = q_dim;

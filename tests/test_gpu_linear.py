@@ -250,18 +250,18 @@ def test_gemm_every_tile(ctx, sa, oracle, tile):
         ctx.set_option(sa.OPT_GEMM_TILE, 0)
 
 
-@pytest.mark.parametrize("tile", range(4, 10), ids=["64x64_8", "64x64_4", "32x64_8", "32x32_4", "16x32_8", "16x16_8"])
-def test_gemm_k_over_waves(ctx, sa, oracle, tile):
-    """k_gemm_kw's configurations forced, at the sizes where they can go wrong:
-    K below one step, not a multiple of a step or of all the waves' steps, and
-    more steps than a wave holds in flight; rows and outputs one past a tile;
-    Q, K and V as segments; the fused norm, activation and residual."""
+@pytest.mark.parametrize("tile", range(3, 9), ids=["64x64", "64x128", "32x64", "32x32", "16x32", "16x16"])
+def test_gemm_staging_waves(ctx, sa, oracle, tile):
+    """k_gemm_sw's configurations forced, at the sizes where they can go wrong:
+    K below one slab, not a multiple of a slab, and more slabs than are held in
+    flight; rows and outputs one past a tile; Q, K and V as segments; the fused
+    norm, activation and residual."""
     ctx.set_option(sa.OPT_GEMM_TILE, tile)
     try:
         for seq, n_in, n_out, has_b, xbf, ybf in [(5, 8, 17, True, False, False), (17, 40, 16, False, True, False),
                                                   (33, 520, 65, True, False, True), (65, 1000, 390, False, False, False),
                                                   (64, 3072, 130, True, True, True), (129, 2048, 64, False, False, False)]:
-            print("gemm kw", tile, seq, n_in, n_out, xbf, ybf, flush=True)
+            print("gemm sw", tile, seq, n_in, n_out, xbf, ybf, flush=True)
             x, w, b = linear_inputs(8700 + n_in + n_out + tile, seq, n_in, n_out, has_b)
             if xbf:
                 xbits = synth.f32_to_bf16_bits(x)
@@ -276,7 +276,7 @@ def test_gemm_k_over_waves(ctx, sa, oracle, tile):
                 g = synth.bf16_bits_to_f32(y.cpu().numpy().view(np.uint16)).astype(np.float64)
                 assert (np.abs(g - ref) <= np.abs(ref) * 2.0 ** -7 + bound(x, w, b)).all()
             else:
-                check(y.cpu().numpy(), ref, x, w, b, "gemm kw %d %s" % (tile, (seq, n_in, n_out)))
+                check(y.cpu().numpy(), ref, x, w, b, "gemm sw %d %s" % (tile, (seq, n_in, n_out)))
         seq, n_in, n_out = 37, 1000, 392
         x, w, b = linear_inputs(8800 + tile, seq, n_in, n_out, True)
         g = (1.0 + 0.1 * synth.normal(8801, (n_in,))).astype(np.float32)
@@ -286,12 +286,57 @@ def test_gemm_k_over_waves(ctx, sa, oracle, tile):
         rd = dev(r)
         sa.linear_ops(ctx, dev(x), dev_bits(w), dev(b), norm_weight=dev(g), eps=1e-6, act=1, residual=rd, out=rd)
         ctx.synchronize()
-        assert_parity(rd.cpu().numpy(), ref, "gemm kw %d ops" % tile)
+        assert_parity(rd.cpu().numpy(), ref, "gemm sw %d ops" % tile)
         ws = [linear_inputs(8810 + i, seq, n_in, n, False)[1] for i, n in enumerate((192, 64, 64))]
         got = sa.linear_qkv_norm(ctx, dev(x), *[dev_bits(v) for v in ws], dev(g), 1e-6)
         ctx.synchronize()
         for y, v in zip(got, ws):
-            assert_parity(y.cpu().numpy(), oracle.linear_bf16(xn, v), "gemm kw %d qkv" % tile)
+            assert_parity(y.cpu().numpy(), oracle.linear_bf16(xn, v), "gemm sw %d qkv" % tile)
+    finally:
+        ctx.set_option(sa.OPT_GEMM_TILE, 0)
+
+
+def _row_products(ctx, sa, x, w, wqkv, g, res, kind):
+    """the projection kinds of a decoder layer over the rows of x"""
+    if kind == "bf16":
+        return [sa.linear(ctx, x, w, out_bf16=True)]
+    if kind == "f32":
+        return [sa.linear_ops(ctx, x, w, residual=res[:x.shape[0]].contiguous())]
+    if kind == "normact":
+        return [sa.linear_ops(ctx, x, w, norm_weight=g, eps=1e-6, act=1)]
+    return list(sa.linear_qkv_norm(ctx, x, *wqkv, g, 1e-6))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f32", "normact", "qkv"])
+@pytest.mark.parametrize("n_in,n_out", [(1024, 1024), (2048, 1024), (3072, 1024), (1024, 6144), (200, 392)])
+def test_gemm_rows_do_not_depend_on_each_other(ctx, sa, kind, n_in, n_out):
+    """A row's projections are the same bits whatever the other rows of the
+    call (more than 4) and whatever tile is forced: every tile forms a sum in
+    one order, so a prompt and its chunks agree."""
+    seq = 700
+    x, w, _ = linear_inputs(9100 + n_in + n_out, seq, n_in, n_out, False)
+    xd, wd = dev(x), dev_bits(w)
+    if kind == "bf16":
+        xd = xd.to(torch.bfloat16)
+    g = dev((1.0 + 0.1 * synth.normal(9101, (n_in,))).astype(np.float32))
+    res = dev(synth.normal(9102, (seq, n_out)))
+    wqkv = [dev_bits(linear_inputs(9110 + i, 5, n_in, n, False)[1]) for i, n in enumerate((256, 128, 128))]
+
+    def run(rows):
+        y = _row_products(ctx, sa, xd[:rows].contiguous(), wd, wqkv, g, res, kind)
+        ctx.synchronize()
+        return [t.cpu() for t in y]
+
+    print("gemm rows", kind, n_in, n_out, flush=True)
+    whole = run(seq)
+    for rows in (5, 16, 26, 64, 130, 333):
+        for a, b in zip(run(rows), whole):
+            assert torch.equal(a, b[:rows]), (kind, rows)
+    try:
+        for tile in range(1, 9):
+            ctx.set_option(sa.OPT_GEMM_TILE, tile)
+            for a, b in zip(run(194), whole):
+                assert torch.equal(a, b[:194]), (kind, tile)
     finally:
         ctx.set_option(sa.OPT_GEMM_TILE, 0)
 
