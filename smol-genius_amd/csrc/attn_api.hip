@@ -679,7 +679,6 @@ struct Plan {
     std::vector<PrepBlock> pblk;
     std::vector<SkBatch> sb;
     std::vector<SkItem> items;
-    int n_groups = 0;
     int q_rows = 0;      /* Q scratch rows per KV head */
     int fresh_rows = 0;  /* fresh rows per KV head */
 };
@@ -747,9 +746,14 @@ static void plan_items(Plan &pl, int Hkv, int G, int window, int rows_per, int c
                 n += std::max(1, ((t.hi - t.lo + SMOL_SLAB - 1) / SMOL_SLAB + per_item - 1) / per_item);
             return n * Hkv;
         };
-        while (pieces(slabs_per_item) > target_items) slabs_per_item++;
+        int hi = slabs_per_item;
+        for (const Tile &t : tiles) hi = std::max(hi, (t.hi - t.lo + SMOL_SLAB - 1) / SMOL_SLAB);
+        while (slabs_per_item < hi) {
+            const int mid = slabs_per_item + (hi - slabs_per_item) / 2;
+            if (pieces(mid) > target_items) slabs_per_item = mid + 1;
+            else hi = mid;
+        }
     }
-    int group = 0;
     const int max_split = SK_MAX_SPLIT;
     for (const Tile &t : tiles) {
         const int n_slabs = (t.hi - t.lo + SMOL_SLAB - 1) / SMOL_SLAB;
@@ -757,28 +761,23 @@ static void plan_items(Plan &pl, int Hkv, int G, int window, int rows_per, int c
         const int n_split = std::min(max_split, want);
         const int per_split = (n_slabs + n_split - 1) / std::max(1, n_split);
         int made = 0;
-        std::vector<SkItem> tmp;
         for (int sp = 0; sp < n_split; sp++) {
             int kb = t.lo + sp * per_split * SMOL_SLAB;
             int ke = std::min(t.hi, kb + per_split * SMOL_SLAB);
             if (sp > 0 && kb >= t.hi) break;
             if (ke < kb) ke = kb;
             const SkBatch &sb = pl.sb[t.batch];
-            tmp.push_back({t.batch, t.row0, kb, ke, group, 0, made++, sb.fresh_row0 - sb.fresh_pos0});
+            pl.items.push_back({t.batch, t.row0, kb, ke, 0, sb.fresh_row0 - sb.fresh_pos0});
+            made++;
         }
-        for (SkItem &it : tmp) {
-            it.n_split = made;
-            pl.items.push_back(it);
-        }
-        group++;
+        for (int k = 1; k <= made; k++) pl.items[pl.items.size() - k].n_split = made;
     }
-    pl.n_groups = group;
 }
 
 /* k_attn_fb with one key group: the tiles (rows_per rows) cut into key
- * pieces, each a work item; the pieces of a tile merge (group = tile, partial
- * slots contiguous). pl.items holds the pieces in slot order, `lists` the
- * pieces of each workgroup of a kv head.
+ * pieces, each a work item; the pieces of a tile merge (partial slots
+ * contiguous). pl.items holds the pieces in slot order; list w of a kv head,
+ * one workgroup's, is the items [starts[w], starts[w + 1]).
  *
  * Fewer tiles than workgroups: each tile is cut into equal pieces, one a
  * workgroup, as long as shorter pieces gain more than the longer merge costs
@@ -787,13 +786,56 @@ static void plan_items(Plan &pl, int Hkv, int G, int window, int rows_per, int c
  * of capacity C in turn, a tile cut exactly where a list is full and
  * continued in the next; a piece costs its slabs plus `overhead` steps
  * (start-up, epilogue), and C is the total cost over the workgroups (raised
- * until the lists fit). Returns the steps that two-group items (64 rows, two
- * slabs a step) of the call would take. */
-static double plan_fb_one(Plan &pl, int Hkv, int G, int window, int rows_per, int cu_count,
-                        std::vector<std::vector<int>> &lists) {
-    const int overhead = 3;
-    struct Tile { int batch, row0, lo, hi, n; };
-    std::vector<Tile> tiles;
+ * until the lists fit). */
+struct FbTile { int batch, row0, lo, hi, n; };
+struct FbOne {
+    static constexpr int overhead = 3;
+    std::vector<FbTile> tiles; /* most slabs first */
+    int rows_per, per;         /* rows of a tile; workgroups of a kv head */
+    int len = 0;               /* slabs of a piece (fewer tiles than workgroups) */
+    double cap = 0;            /* or the lists' capacity */
+    double one = 0;            /* steps of the longest list */
+    double two = 0;            /* steps that two-group items (64 rows, two slabs a step) would take */
+};
+
+/* the pieces of every tile in turn: f(tile, first slab, slabs, list); false
+ * when a tile would be cut into more than SK_MAX_SPLIT */
+template <class F> static bool fb_one_pieces(const FbOne &o, double cap, F f) {
+    int list = 0;
+    if (o.len > 0) {
+        for (int t = 0; t < (int)o.tiles.size(); t++) {
+            const int n = o.tiles[t].n, ns = std::max(1, (n + o.len - 1) / o.len);
+            const int len = std::max(1, (n + ns - 1) / ns);
+            for (int first = 0; first == 0 || first < n; first += len) f(t, first, std::min(len, n - first), list++);
+        }
+        return true;
+    }
+    double room = cap;
+    bool empty = true;
+    for (int t = 0; t < (int)o.tiles.size(); t++) {
+        const int n = o.tiles[t].n;
+        int first = 0, made = 0;
+        do {
+            if (room < FbOne::overhead + 1 && !empty) {
+                list++;
+                empty = true;
+                room = cap;
+            }
+            const int take = std::min(n - first, std::max(1, (int)(room - FbOne::overhead)));
+            f(t, first, take, list);
+            empty = false;
+            first += take;
+            room -= take + FbOne::overhead;
+            if (++made > SK_MAX_SPLIT) return false;
+        } while (first < n);
+    }
+    return true;
+}
+
+static FbOne plan_fb_one(const Plan &pl, int Hkv, int G, int window, int rows_per, int cu_count) {
+    FbOne o;
+    o.rows_per = rows_per;
+    o.per = std::max(1, cu_count / std::max(1, Hkv));
     long long total = 0;
     int longest = 1;
     for (int bi = 0; bi < (int)pl.sb.size(); bi++) {
@@ -807,84 +849,78 @@ static double plan_fb_one(Plan &pl, int Hkv, int G, int window, int rows_per, in
             }
             lo = std::max(lo, 0) & ~(SMOL_SLAB - 1);
             const int n = hi > lo ? (hi - lo + SMOL_SLAB - 1) / SMOL_SLAB : 0;
-            tiles.push_back({bi, r0, lo, std::max(hi, lo), n});
-            total += n + overhead;
+            o.tiles.push_back({bi, r0, lo, std::max(hi, lo), n});
+            total += n + FbOne::overhead;
             longest = std::max(longest, n);
         }
     }
-    std::stable_sort(tiles.begin(), tiles.end(), [](const Tile &a, const Tile &b) { return a.n > b.n; });
-    const int per = std::max(1, cu_count / std::max(1, Hkv)); /* workgroups of a kv head */
-    const double two = std::max(longest / 2.0, (double)total / (rows_per / 64) / per);
-    const int n_tiles = (int)tiles.size();
-    struct Piece { int tile, first, count; };
-    std::vector<std::vector<Piece>> bins;
-    if (n_tiles <= per) {
-        int best = longest;
-        double best_c = longest;
-        for (int len = longest - 1; len >= 1; len--) {
+    std::stable_sort(o.tiles.begin(), o.tiles.end(), [](const FbTile &a, const FbTile &b) { return a.n > b.n; });
+    const int per = o.per;
+    o.two = std::max(longest / 2.0, (double)total / (rows_per / 64) / per);
+    if ((int)o.tiles.size() <= per) {
+        /* the shortest pieces that are no more than the workgroups (their
+         * number falls as they get longer) */
+        auto pieces = [&](int len) {
             long long n = 0;
-            for (const Tile &t : tiles) n += std::max(1, (t.n + len - 1) / len);
-            const int ns = (longest + len - 1) / len;
-            if (n > per || ns > SK_MAX_SPLIT) break;
+            for (const FbTile &t : o.tiles) n += std::max(1, (t.n + len - 1) / len);
+            return n;
+        };
+        int lo = std::max(1, (longest + SK_MAX_SPLIT - 1) / SK_MAX_SPLIT), hi = longest;
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (pieces(mid) <= per) hi = mid;
+            else lo = mid + 1;
+        }
+        /* the longest tile in ns pieces: the shortest such length is the best */
+        o.len = longest;
+        double best = longest;
+        for (int ns = 2; ns <= SK_MAX_SPLIT; ns++) {
+            const int len = std::max(lo, (longest + ns - 1) / ns);
+            if ((longest + len - 1) / len != ns) continue;
             const double cost = len + 3 + 0.1 * ns;
-            if (cost < best_c) {
-                best_c = cost;
-                best = len;
+            if (cost < best) {
+                best = cost;
+                o.len = len;
             }
         }
-        for (int t = 0; t < n_tiles; t++) {
-            const int ns = std::max(1, (tiles[t].n + best - 1) / best);
-            const int len = std::max(1, (tiles[t].n + ns - 1) / ns);
-            for (int first = 0; first == 0 || first < tiles[t].n; first += len)
-                bins.push_back({{t, first, std::min(len, tiles[t].n - first)}});
+        for (const FbTile &t : o.tiles) {
+            const int ns = std::max(1, (t.n + o.len - 1) / o.len);
+            o.one = std::max(o.one, (double)((t.n + ns - 1) / ns));
         }
-    } else {
-        for (double cap = std::max(1.0, (double)total / per);; cap *= 1.02) {
-            bins.assign(1, {});
-            double room = cap;
-            bool ok = true;
-            for (int t = 0; t < n_tiles && ok; t++) {
-                int first = 0, made = 0;
-                do {
-                    if (room < overhead + 1 && !bins.back().empty()) {
-                        bins.push_back({});
-                        room = cap;
-                    }
-                    const int take = std::min(tiles[t].n - first, std::max(1, (int)(room - overhead)));
-                    bins.back().push_back({t, first, take});
-                    first += take;
-                    room -= take + overhead;
-                    if (++made > SK_MAX_SPLIT) ok = false;
-                } while (first < tiles[t].n);
-            }
-            if (ok && (int)bins.size() <= per) break;
-        }
+        return o;
     }
-    /* items in slot order: a tile's pieces contiguous, in key order */
-    struct Placed { int first, count, list; };
-    std::vector<std::vector<Placed>> of(tiles.size());
-    for (int w = 0; w < (int)bins.size(); w++)
-        for (const Piece &pc : bins[w]) of[pc.tile].push_back({pc.first, pc.count, w});
-    lists.assign(bins.size(), {});
-    pl.items.clear();
-    for (int t = 0; t < (int)tiles.size(); t++) {
-        const Tile &tl = tiles[t];
-        const SkBatch &sb = pl.sb[tl.batch];
-        std::sort(of[t].begin(), of[t].end(), [](const Placed &a, const Placed &b) { return a.first < b.first; });
-        const int ns = (int)of[t].size();
-        for (int sp = 0; sp < ns; sp++) {
-            const Placed &pc = of[t][sp];
-            const int kb = tl.lo + pc.first * SMOL_SLAB;
-            const int ke = sp == ns - 1 ? tl.hi : tl.lo + (pc.first + pc.count) * SMOL_SLAB;
-            lists[pc.list].push_back((int)pl.items.size());
-            pl.items.push_back({tl.batch, tl.row0, kb, std::max(kb, ke), t, ns, sp, sb.fresh_row0 - sb.fresh_pos0});
-        }
+    for (o.cap = std::max(1.0, (double)total / per);; o.cap *= 1.02) {
+        int lists = 0, at = -1;
+        double steps = 0;
+        o.one = 0;
+        const bool ok = fb_one_pieces(o, o.cap, [&](int, int, int take, int list) {
+            steps = list == at ? steps + take + FbOne::overhead : take;
+            at = list;
+            lists = list + 1;
+            o.one = std::max(o.one, steps);
+        });
+        if (ok && lists <= per) return o;
     }
-    pl.n_groups = (int)tiles.size();
-    return two;
 }
 
-/* the pre-pass blocks with their batches */
+static void build_fb_one(Plan &pl, const FbOne &o, std::vector<int> &starts) {
+    int made = 0; /* pieces of the tile so far */
+    fb_one_pieces(o, o.cap, [&](int t, int first, int take, int list) {
+        const FbTile &tl = o.tiles[t];
+        const SkBatch &sb = pl.sb[tl.batch];
+        if (list == (int)starts.size()) starts.push_back((int)pl.items.size());
+        const bool last = first + take >= tl.n;
+        const int kb = tl.lo + first * SMOL_SLAB;
+        const int ke = last ? tl.hi : tl.lo + (first + take) * SMOL_SLAB;
+        pl.items.push_back({tl.batch, tl.row0, kb, std::max(kb, ke), 0, sb.fresh_row0 - sb.fresh_pos0});
+        made++;
+        if (!last) return;
+        for (int k = 1; k <= made; k++) pl.items[pl.items.size() - k].n_split = made;
+        made = 0;
+    });
+    starts.push_back((int)pl.items.size());
+}
+
 /* the pre-pass blocks with their batches; without_q: the Q blocks are left
  * out (k_attn_fb prepares its Q rows itself). A fresh slab becomes two
  * blocks, its K and its V (count 1 and 2), when the launch then still fits
@@ -913,12 +949,13 @@ static std::vector<PrepBlockB> prep_records(const Plan &pl, bool without_q, int 
 }
 
 /* k_attn_fb items with their batches' fields. With n_wg > 0 (fewer
- * workgroups per kv head than items) each item, longest first, goes to the
- * list with the least work so far: an item costs its steps (two slabs each,
- * one per key group) plus about six steps of start-up and epilogue. Item w
- * heads list w; `next` links the rest. */
-static std::vector<FbItem> fb_items(const Plan &pl, int n_wg, bool one_group,
-                                    const std::vector<std::vector<int>> *given = nullptr) {
+ * workgroups per kv head than items) item w heads workgroup w's list and
+ * `next` links the rest. `starts`: list w is the items [starts[w],
+ * starts[w + 1]) (build_fb_one). Without it (two key groups) each item,
+ * longest first, goes to the list with the least work so far: an item costs
+ * its steps (two slabs each, one per key group) plus about six steps of
+ * start-up and epilogue. */
+static std::vector<FbItem> fb_items(const Plan &pl, int n_wg, const std::vector<int> *starts = nullptr) {
     const int n = (int)pl.items.size();
     auto record = [&](int i) {
         const SkItem &it = pl.items[i];
@@ -928,9 +965,7 @@ static std::vector<FbItem> fb_items(const Plan &pl, int n_wg, bool one_group,
         f.key_begin = it.key_begin; f.key_end = it.key_end; f.fresh_off = it.fresh_off; f.row0 = it.row0;
         f.n_rows = b.n_rows; f.q_row0 = b.q_row0; f.out_tok0 = b.out_tok0; f.q_pos0 = b.q_pos0;
         f.key_lo = b.key_lo; f.key_hi = b.key_hi; f.causal = b.causal; f.next = -1;
-        /* merge group and partial slot: a group's items are contiguous in
-         * the plan, so slot i - split is the group's first */
-        f.group = it.group; f.n_split = it.n_split; f.split = it.split; f.part = i;
+        f.n_split = it.n_split; f.part = i; /* the partial slot */
         return f;
     };
     std::vector<FbItem> out(n);
@@ -938,43 +973,42 @@ static std::vector<FbItem> fb_items(const Plan &pl, int n_wg, bool one_group,
         for (int i = 0; i < n; i++) out[i] = record(i);
         return out;
     }
-    std::vector<std::vector<int>> lists;
-    if (given) {
-        lists = *given; /* the planner's lists (plan_fb_fill) */
-        n_wg = (int)lists.size();
-    } else {
+    /* the heads first, then the rest list by list */
+    int k = n_wg;
+    if (starts) {
+        for (int w = 0; w < n_wg; w++) {
+            int at = w;
+            for (int i = (*starts)[w]; i < (*starts)[w + 1]; i++) {
+                out[at] = record(i);
+                if (i + 1 < (*starts)[w + 1]) at = out[at].next = k++;
+            }
+        }
+        return out;
+    }
+    std::vector<std::vector<int>> lists(n_wg);
     std::vector<int> order(n);
     for (int i = 0; i < n; i++) order[i] = i;
     auto cost = [&](int i) {
         const SkItem &it = pl.items[i];
-        const int slabs = (it.key_end - it.key_begin + SMOL_SLAB - 1) / SMOL_SLAB;
-        /* a step per slab (one key group) or per two (two groups), start-up
-         * and epilogue, and a publish and merge for a split item */
-        return one_group ? slabs + 6 + (it.n_split > 1 ? 2 : 0) : (slabs + 1) / 2 + 6;
+        return ((it.key_end - it.key_begin + SMOL_SLAB - 1) / SMOL_SLAB + 1) / 2 + 6;
     };
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
     using Load = std::pair<long long, int>; /* (work, list) */
     std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
     for (int w = 0; w < n_wg; w++) heap.push({0, w});
-    lists.assign(n_wg, {});
     for (int i : order) {
         Load l = heap.top();
         heap.pop();
         lists[l.second].push_back(i);
         heap.push({l.first + cost(i), l.second});
     }
-    }
-    /* new index of every item: the heads first, then the rest list by list */
-    std::vector<int> at(n, -1);
-    int k = n_wg;
-    for (int w = 0; w < n_wg; w++)
-        for (size_t e = 0; e < lists[w].size(); e++) at[lists[w][e]] = e == 0 ? w : k++;
-    for (int w = 0; w < n_wg; w++)
+    for (int w = 0; w < n_wg; w++) {
+        int at = w;
         for (size_t e = 0; e < lists[w].size(); e++) {
-            FbItem f = record(lists[w][e]);
-            if (e + 1 < lists[w].size()) f.next = at[lists[w][e + 1]];
-            out[at[lists[w][e]]] = f;
+            out[at] = record(lists[w][e]);
+            if (e + 1 < lists[w].size()) at = out[at].next = k++;
         }
+    }
     return out;
 }
 
@@ -1353,23 +1387,14 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
      * leave workgroups idle. Measured, two groups / one (us): 500 rows on
      * 2048 keys, 8 kv heads, 49 / 34; 256 on 1024 26.7 / 21; 1000 on 500 34.7
      * / 35.8; 300 in a window of 512 19 / 22; 1536 on none 36.6 / 45. */
-    std::vector<std::vector<int>> fill_lists;
+    std::vector<int> list_starts;
     const int fbg = ctx->opt[SMOL_OPT_FB_GROUPS];
     bool fb_one = fb && (hd > 128 || (fbg != 2 && ctx->opt[SMOL_OPT_FB_NT] != 2));
     if (fb_one) {
         rows_per = hd > 128 ? 64 : 128;
-        const double two = plan_fb_one(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count, fill_lists);
-        double one = 0;
-        for (const auto &l : fill_lists) {
-            double slabs = 3.0 * (l.size() - 1);
-            for (int i : l) slabs += (pl.items[i].key_end - pl.items[i].key_begin + SMOL_SLAB - 1) / SMOL_SLAB;
-            one = std::max(one, slabs);
-        }
-        fb_one = hd > 128 || fbg == 1 || one + 8 < two;
-        if (!fb_one) {
-            pl.items.clear();
-            fill_lists.clear();
-        }
+        const FbOne o = plan_fb_one(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count);
+        fb_one = hd > 128 || fbg == 1 || o.one + 8 < o.two;
+        if (fb_one) build_fb_one(pl, o, list_starts);
     }
     if (fb_one) {
         nt = 0; /* the launcher's code for one key group */
@@ -1432,10 +1457,10 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     if (!((int)n_items > fb_wg && ctx->opt[SMOL_OPT_FB_LISTS] != -1)) fb_wg = 0;
     if (fb_one) {
         /* one key group: the planner's lists, one workgroup each */
-        fb_wg = (int)fill_lists.size();
-        fbi = fb_items(pl, fb_wg, true, &fill_lists);
+        fb_wg = (int)list_starts.size() - 1;
+        fbi = fb_items(pl, fb_wg, &list_starts);
     } else if (fb) {
-        fbi = fb_items(pl, fb_wg, fb_one);
+        fbi = fb_items(pl, fb_wg);
     }
 
     /* descriptor tables in one upload: pre-pass blocks and items, each with

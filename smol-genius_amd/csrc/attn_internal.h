@@ -55,9 +55,7 @@ typedef struct {
     int row0;        /* first row (within the batch) of this item's row tiles */
     int key_begin;   /* slab-aligned */
     int key_end;
-    int group;       /* merge group id (one output row tile) */
-    int n_split;     /* items in the group */
-    int split;       /* index of this item in its group */
+    int n_split;     /* items of the row tile (its merge group) */
     int fresh_off;   /* the batch's fresh_row0 - fresh_pos0: fresh row of key k is k + fresh_off */
 } SkItem;
 
@@ -78,7 +76,7 @@ typedef struct {
     int key_begin, key_end, fresh_off, row0;
     int n_rows, q_row0, out_tok0, q_pos0;
     int key_lo, key_hi, causal, next;
-    int group, n_split, split, part;
+    int n_split, part;
 } FbItem;
 
 /* A row tile whose keys were split over several items (k_sk_merge): its

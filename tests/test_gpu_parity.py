@@ -3,6 +3,8 @@
 Every case prints its name before it runs. The bar is |gpu - cpu| <= 2e-3 +
 1e-2 |cpu| for every element (conftest.ATOL / RTOL), on fp32 outputs.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -518,6 +520,42 @@ def test_prefill_staged_prefix(ctx, sa, oracle, wo, opts, hq, hkv, hd):
             if not window and not cap:
                 assert_parity(got, wo.prefill(oracle, wl, x), "staged prefix %s P=%d S=%d" % (name, P, S))
             assert np.linalg.norm(got - fa) <= 1e-5 * np.linalg.norm(fa), (name, P, S, window, cap)
+
+
+def _prefill_with(sa, ctx, wl, x, window=0, calls=1):
+    """one prefill's output on a new cache, and the host's us a call over `calls` more"""
+    kv = sa.KVCache(ctx, 1, 1, wl.Hkv, wl.hd, wl.pos0 + wl.seq_q)
+    if wl.pos0:
+        kv.write(0, 0, 0, x["cache_k"], x["cache_v"])
+    rope = sa.RopeTable(ctx, wl.hd, wl.theta, 0)
+    q, k, v = dev(x["q"]), dev(x["k"]), dev(x["v"])
+    call = sa.prefill_call(ctx, kv, 0, 0, rope, wl.pos0, q, k, v, wl.Hq, wl.scale, window=window)
+    call()
+    ctx.synchronize()
+    out = call.out.cpu().numpy()
+    host = []
+    for _ in range(calls):
+        t = time.perf_counter()
+        call()
+        host.append(time.perf_counter() - t)
+        ctx.synchronize()
+    return out, 1e6 * float(np.median(host))
+
+
+@pytest.mark.parametrize("hq,hkv,hd,P,S,window", [(8, 1, 256, 0, 2500, 512), (8, 1, 256, 2000, 1000, 0)])
+def test_prefill_planning_time(sa, ctx, opts, hq, hkv, hd, P, S, window):
+    """Planning a call for k_attn_fb on the host takes no more than three times
+    what it takes for k_attn_fa, whose plan is one pass over the tiles (it took
+    six times that when every capacity of the lists was laid out in full)."""
+    from smol_genius_amd.workloads import Prefill
+    print("prefill planning", hq, hkv, hd, P, S, window, flush=True)
+    wl = Prefill("t", hq, hkv, hd, P, S, 1e5, seed=721, in_bf16=False)
+    x = wl.inputs()
+    _, fb = _prefill_with(sa, ctx, wl, x, window, calls=15)
+    opts(sa.OPT_PREFILL_KERNEL, 2)
+    _, fa = _prefill_with(sa, ctx, wl, x, window, calls=15)
+    print("host us a call: k_attn_fb %.1f, k_attn_fa %.1f" % (fb, fa), flush=True)
+    assert fb <= 3 * fa
 
 
 @pytest.mark.parametrize("window,cap", [(16, 0.0), (0, 2.0), (1, 0.0), (40, 1.5), (1, 3.0)])
