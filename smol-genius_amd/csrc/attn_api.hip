@@ -795,7 +795,8 @@ struct FbOne {
     int len = 0;               /* slabs of a piece (fewer tiles than workgroups) */
     double cap = 0;            /* or the lists' capacity */
     double one = 0;            /* steps of the longest list */
-    double two = 0;            /* steps that two-group items (64 rows, two slabs a step) would take */
+    int split_pieces = 0;      /* pieces of tiles that are cut */
+    double two = 0;            /* steps of the longest list of two-group items (64 rows, two slabs a step) */
 };
 
 /* the pieces of every tile in turn: f(tile, first slab, slabs, list); false
@@ -836,10 +837,11 @@ static FbOne plan_fb_one(const Plan &pl, int Hkv, int G, int window, int rows_pe
     FbOne o;
     o.rows_per = rows_per;
     o.per = std::max(1, cu_count / std::max(1, Hkv));
-    long long total = 0;
-    int longest = 1;
+    long long total = 0, slabs = 0;
+    int longest = 1, n64 = 0; /* 64-row tiles */
     for (int bi = 0; bi < (int)pl.sb.size(); bi++) {
         const SkBatch &b = pl.sb[bi];
+        n64 += (b.n_rows + 63) / 64;
         for (int r0 = 0; r0 < b.n_rows; r0 += rows_per) {
             const int r1 = std::min(r0 + rows_per, b.n_rows) - 1;
             int lo = b.key_lo, hi = b.key_hi;
@@ -851,12 +853,21 @@ static FbOne plan_fb_one(const Plan &pl, int Hkv, int G, int window, int rows_pe
             const int n = hi > lo ? (hi - lo + SMOL_SLAB - 1) / SMOL_SLAB : 0;
             o.tiles.push_back({bi, r0, lo, std::max(hi, lo), n});
             total += n + FbOne::overhead;
+            slabs += n;
             longest = std::max(longest, n);
         }
     }
     std::stable_sort(o.tiles.begin(), o.tiles.end(), [](const FbTile &a, const FbTile &b) { return a.n > b.n; });
     const int per = o.per;
-    o.two = std::max(longest / 2.0, (double)total / (rows_per / 64) / per);
+    /* a 64-row item takes half its tile's slabs in steps, and six more where
+     * its workgroup's list goes on: the longest item, the lists' average, or
+     * the two items that meet first when the longest go to lists of their own */
+    auto half = [&](int t) { return (o.tiles[t].n + 1) / 2; };
+    o.two = (longest + 1) / 2;
+    if (n64 > per && rows_per == 128) {
+        o.two = std::max(o.two, (double)(slabs + 13 * (long long)o.tiles.size()) / per - 6);
+        if (per / 2 < (int)o.tiles.size()) o.two = std::max(o.two, half((per - 1) / 2) + half(per / 2) + 6.0);
+    }
     if ((int)o.tiles.size() <= per) {
         /* the shortest pieces that are no more than the workgroups (their
          * number falls as they get longer) */
@@ -886,6 +897,7 @@ static FbOne plan_fb_one(const Plan &pl, int Hkv, int G, int window, int rows_pe
         for (const FbTile &t : o.tiles) {
             const int ns = std::max(1, (t.n + o.len - 1) / o.len);
             o.one = std::max(o.one, (double)((t.n + ns - 1) / ns));
+            if (ns > 1) o.split_pieces += ns;
         }
         return o;
     }
@@ -893,11 +905,13 @@ static FbOne plan_fb_one(const Plan &pl, int Hkv, int G, int window, int rows_pe
         int lists = 0, at = -1;
         double steps = 0;
         o.one = 0;
-        const bool ok = fb_one_pieces(o, o.cap, [&](int, int, int take, int list) {
+        o.split_pieces = 0;
+        const bool ok = fb_one_pieces(o, o.cap, [&](int t, int, int take, int list) {
             steps = list == at ? steps + take + FbOne::overhead : take;
             at = list;
             lists = list + 1;
             o.one = std::max(o.one, steps);
+            o.split_pieces += take < o.tiles[t].n;
         });
         if (ok && lists <= per) return o;
     }
@@ -1358,10 +1372,9 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     const int G = cs.Hq / cs.Hkv;
     int max_rows = 0;
     for (auto &b : pl.sb) max_rows = std::max(max_rows, b.n_rows);
-    /* prefill kernel: k_attn_fb (one workgroup per 64-row tile, no merges
-     * between workgroups) when every key is in the fresh buffers and the
-     * call has enough tiles to occupy the device, else k_attn_fa (waves
-     * split the rows, K/V shared through LDS, split-K across workgroups);
+    /* prefill kernel: k_attn_fb when every key is in the fresh buffers and the
+     * call has more than a few short tiles, else k_attn_fa (waves split the
+     * rows, K/V shared through LDS, split-K across workgroups);
      * SMOL_OPT_PREFILL_KERNEL forces one where the keys allow it */
     const int pk = ctx->opt[SMOL_OPT_PREFILL_KERNEL];
     const bool precise = ctx->opt[SMOL_OPT_QK_FP16] != 1;
@@ -1369,31 +1382,48 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     bool fb = fa && pk != 2;
     if (fb) {
         long long tiles = 0;
+        int keys = 0; /* that a row tile may see */
         bool widened = false; /* cache rows staged as fresh ones (smol_attn_prefill) */
         for (auto &b : pl.sb) {
             if (b.key_lo < b.fresh_pos0) fb = false;
             widened |= b.slot >= 0 && b.fresh_pos0 < (b.q_pos0 & ~(SMOL_SLAB - 1));
             tiles += (b.n_rows + 63) / 64;
+            const int lo = b.causal && cs.window > 0 ? std::max(b.key_lo, b.q_pos0 - cs.window + 1) : b.key_lo;
+            keys = std::max(keys, b.key_hi - lo);
         }
-        if (pk != 1 && hd <= 128 && !widened && tiles * cs.Hkv < ctx->cu_count / 4) fb = false;
+        /* up to four tiles of at most four slabs: k_attn_fa, which does not cut them
+         * (100 tokens, 8 kv heads: 15.3 us, k_attn_fb 15.9). Longer ones it
+         * cuts, and the merge's launch then costs more than k_attn_fb's two key
+         * groups (131 keys: 18.8 / 16; 300 of 4 kv heads at head_dim 64 18.8 /
+         * 15.3) */
+        if (pk != 1 && hd <= 128 && !widened && tiles <= 4 && tiles * cs.Hkv < ctx->cu_count / 4 &&
+            keys <= 4 * SMOL_SLAB)
+            fb = false;
     }
     int nt = 1, w = 2, rows_per = 64;
     /* k_attn_fb with two key groups (64-row items, each group half of the
      * keys, nothing to merge outside the workgroup) or one key group of eight
      * waves (128-row items whose keys may be split over workgroups; at
-     * head_dim 256 always: four waves, 64-row items). Where one key group's
-     * longest list of slabs and eight steps more (writing partials, the merge
-     * launch) are below the two-group items' steps: few long tiles, which
-     * leave workgroups idle. Measured, two groups / one (us): 500 rows on
+     * head_dim 256 always: four waves, 64-row items), whichever should take
+     * fewer steps. A one-group step (128 rows, one slab) takes 0.85 of a
+     * two-group one; lists that cut tiles take a quarter more than their
+     * slabs say; writing partials and the merge's launch take nine steps and
+     * four more for every 256 pieces. Fitted to 1208 measured calls (head_dim
+     * 64, 72, 96 and 128; 40 to 2000 rows on 0 to 6000 keys, with and without
+     * a window of 512): within 0.2% of the better form on average, one group
+     * taken where it is slower by 3.2% at most. Two groups / one (us): 500 rows on
      * 2048 keys, 8 kv heads, 49 / 34; 256 on 1024 26.7 / 21; 1000 on 500 34.7
-     * / 35.8; 300 in a window of 512 19 / 22; 1536 on none 36.6 / 45. */
+     * / 35.8; 1536 on none 36.6 / 45; head_dim 64, 4 kv heads, 1000 rows on
+     * none 24 / 26, 2000 in a window of 512 20.4 / 22.2; head_dim 128, 32
+     * heads over 4, 1000 rows in a window of 512 42 / 31. */
     std::vector<int> list_starts;
     const int fbg = ctx->opt[SMOL_OPT_FB_GROUPS];
     bool fb_one = fb && (hd > 128 || (fbg != 2 && ctx->opt[SMOL_OPT_FB_NT] != 2));
     if (fb_one) {
         rows_per = hd > 128 ? 64 : 128;
         const FbOne o = plan_fb_one(pl, cs.Hkv, G, cs.window, rows_per, ctx->cu_count);
-        fb_one = hd > 128 || fbg == 1 || o.one + 8 < o.two;
+        const double cut = o.split_pieces > 0 ? 9 + 4.0 * o.split_pieces * cs.Hkv / 256 : 0;
+        fb_one = hd > 128 || fbg == 1 || 0.85 * o.one * (o.len == 0 && cut > 0 ? 1.25 : 1) + cut < o.two;
         if (fb_one) build_fb_one(pl, o, list_starts);
     }
     if (fb_one) {
@@ -1663,7 +1693,9 @@ extern "C" int smol_attn_prefill_qknorm(smol_attn_ctx *ctx, smol_kv_cache *kv, i
     if ((rc = check_rope(ctx, rope, kv->hd, pos0 + seq_q))) return rc;
     const int Hkv = kv->n_kv, G = n_heads / Hkv, hd = kv->hd;
     Plan pl;
-    /* More than 128 rows (head_dim 256: any): the pre-pass also stages the
+    /* More than 128 rows (head_dim 256: any; fewer rows where k_attn_fa would
+     * cut the few keys, 129 to 512 of them, and merge: 66 tokens of 8 heads at
+     * head_dim 64 on 64 to 200 keys 16.5 / 12): the pre-pass also stages the
      * cache rows that the call can see, widened to fp16, and k_attn_fb reads
      * every key from there. That costs 4 bytes read and 6 written per key
      * and element (8000 keys of 8 heads: 11 us); k_attn_fb's slab step, staged by
@@ -1673,7 +1705,9 @@ extern "C" int smol_attn_prefill_qknorm(smol_attn_ctx *ctx, smol_kv_cache *kv, i
      * 60 / 44; head_dim 256, 100 tokens on 1000 38 / 31). The staging stays
      * below 6 bytes x 32768 keys x n_kv x head_dim. */
     const int pk = ctx->opt[SMOL_OPT_PREFILL_KERNEL];
-    const bool widen = seq_q * G > 64 && pk != 2 && (pk == 1 || hd > 128 || seq_q * G > 128) && pos0 <= 32768;
+    const int seen = pos0 + seq_q - (window > 0 ? std::max(0, pos0 - window + 1) : 0);
+    const bool few_keys = seen > 4 * SMOL_SLAB && seen <= 512;
+    const bool widen = seq_q * G > 64 && pk != 2 && (pk == 1 || hd > 128 || seq_q * G > 128 || few_keys) && pos0 <= 32768;
     const int f0 = (widen ? (window > 0 ? std::max(0, pos0 - window + 1) : 0) : pos0) & ~(SMOL_SLAB - 1);
     const int nf = ((pos0 + seq_q + SMOL_SLAB - 1) & ~(SMOL_SLAB - 1)) - f0;
     pl.pb.push_back({0, seq_q, 0, pos0, 0, seq_q, pos0, f0, nf, 0, slot, 0});

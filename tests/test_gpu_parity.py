@@ -542,6 +542,27 @@ def _prefill_with(sa, ctx, wl, x, window=0, calls=1):
     return out, 1e6 * float(np.median(host))
 
 
+@pytest.mark.parametrize("hq,hkv,hd,P,S,window,form", [
+    (8, 4, 64, 0, 1000, 0, 2), (8, 4, 64, 0, 2000, 512, 2), (8, 4, 64, 0, 300, 0, 2), (8, 8, 64, 100, 66, 0, 2),
+    (16, 8, 128, 31, 100, 0, 2), (16, 8, 128, 2048, 500, 0, 1), (32, 4, 128, 0, 1000, 512, 1)])
+def test_prefill_form_chosen(sa, ctx, opts, hq, hkv, hd, P, S, window, form):
+    """k_attn_fb runs each call in the form that measures faster (one key
+    group's merge costs a launch, which short key ranges do not earn back; nor
+    do those of k_attn_fa): the bits of the form forced. The two forms add in
+    other orders, so their bits tell them apart."""
+    from smol_genius_amd.workloads import Prefill
+    print("prefill form", hq, hkv, hd, P, S, window, flush=True)
+    wl = Prefill("t", hq, hkv, hd, P, S, 1e5, seed=720 + S, in_bf16=False)
+    x = wl.inputs()
+    auto, _ = _prefill_with(sa, ctx, wl, x, window)
+    opts(sa.OPT_PREFILL_KERNEL, 1)
+    opts(sa.OPT_FB_GROUPS, form)
+    want, _ = _prefill_with(sa, ctx, wl, x, window)
+    opts(sa.OPT_FB_GROUPS, 3 - form)
+    other, _ = _prefill_with(sa, ctx, wl, x, window)
+    assert np.array_equal(auto, want) and not np.array_equal(auto, other)
+
+
 @pytest.mark.parametrize("hq,hkv,hd,P,S,window", [(8, 1, 256, 0, 2500, 512), (8, 1, 256, 2000, 1000, 0)])
 def test_prefill_planning_time(sa, ctx, opts, hq, hkv, hd, P, S, window):
     """Planning a call for k_attn_fb on the host takes no more than three times
