@@ -113,7 +113,8 @@ SMOL_ATTN_API int smol_attn_ctx_timing_read(smol_attn_ctx *ctx, double *ms, int 
  * tolerance whatever they are set to, except under SMOL_OPT_FAULT_MERGE,
  * which exists to test the error path. */
 #define SMOL_OPT_PREFILL_KERNEL 0 /* 1: k_attn_fb wherever its keys allow, 2: k_attn_fa */
-#define SMOL_OPT_FB_LISTS 1       /* -1: one k_attn_fb workgroup per tile (no tile lists) */
+#define SMOL_OPT_FB_LISTS 1       /* -1: one k_attn_fb workgroup per tile, or per piece of one whose keys are split
+                                   * (no lists) */
 #define SMOL_OPT_FB_NT 2          /* 2: two row tiles per k_attn_fb wave */
 #define SMOL_OPT_DEC_SLABS 3      /* k_dec: 32-key slabs per workgroup (0: by call size) */
 #define SMOL_OPT_DEC_WAVES 4      /* k_dec: 4 or 8 waves per workgroup (0: by shape) */
@@ -145,7 +146,9 @@ SMOL_ATTN_API int smol_attn_ctx_timing_read(smol_attn_ctx *ctx, double *ms, int 
 #define SMOL_OPT_FB_QPREP 14      /* k_attn_fb at head_dim 64 / 128 with precise QK^T and no per-head
                                    * Q norm: 0: each item rotates and scales its own Q rows from the
                                    * inputs; 1: the pre-pass stages them (as for k_attn_fa) */
-#define SMOL_OPT_COUNT 15
+#define SMOL_OPT_FB_WORKGROUPS 15 /* read only: workgroups per kv head of the context's last k_attn_fb launch (0:
+                                   * none yet) */
+#define SMOL_OPT_COUNT 16
 SMOL_ATTN_API int smol_attn_ctx_set_option(smol_attn_ctx *ctx, int option, int value);
 SMOL_ATTN_API int smol_attn_ctx_get_option(smol_attn_ctx *ctx, int option, int *value);
 

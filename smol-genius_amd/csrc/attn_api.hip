@@ -451,7 +451,8 @@ extern "C" void *smol_attn_ctx_stream(smol_attn_ctx *ctx) { return ctx ? (void *
 
 extern "C" int smol_attn_ctx_set_option(smol_attn_ctx *ctx, int option, int value) {
     if (!ctx) return fail(SMOL_ATTN_ERR_ARG, "ctx is NULL");
-    if (option < 0 || option >= SMOL_OPT_COUNT || option == SMOL_OPT_XCD_CHECK)
+    if (option < 0 || option >= SMOL_OPT_COUNT || option == SMOL_OPT_XCD_CHECK ||
+        option == SMOL_OPT_FB_WORKGROUPS)
         return fail(SMOL_ATTN_ERR_ARG, "option %d cannot be set", option);
     ctx->opt[option] = value;
     return SMOL_ATTN_OK;
@@ -1485,13 +1486,14 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     std::vector<FbItem> fbi;
     int fb_wg = std::max(1, ctx->cu_count / cs.Hkv);
     if (!((int)n_items > fb_wg && ctx->opt[SMOL_OPT_FB_LISTS] != -1)) fb_wg = 0;
-    if (fb_one) {
+    if (fb_one && ctx->opt[SMOL_OPT_FB_LISTS] != -1) {
         /* one key group: the planner's lists, one workgroup each */
         fb_wg = (int)list_starts.size() - 1;
         fbi = fb_items(pl, fb_wg, &list_starts);
     } else if (fb) {
         fbi = fb_items(pl, fb_wg);
     }
+    if (fb) ctx->opt[SMOL_OPT_FB_WORKGROUPS] = fb_wg > 0 ? fb_wg : (int)n_items;
 
     /* descriptor tables in one upload: pre-pass blocks and items, each with
      * its batch */

@@ -477,11 +477,44 @@ def test_fb_one_key_group(ctx, sa, oracle, case, qk_fp16, opts):
     """k_attn_fb with one key group of eight waves (SMOL_OPT_FB_GROUPS 1):
     128-row items whose long key ranges are split over workgroups and merged
     by k_sk_merge. The same cases as the tile lists, with both
-    QK^T modes; with lists and with one workgroup per item the merges add the
+    QK^T modes; with lists and with one workgroup per piece the merges add the
     same partials in the same order, so the two launches agree bit for bit."""
     opts(sa.OPT_FB_GROUPS, 1)
     opts(sa.OPT_QK_FP16, qk_fp16)
     test_fb_tile_lists(ctx, sa, oracle, case, opts)
+
+
+@pytest.mark.parametrize("hd,P,S,window", [(256, 0, 1100, 0), (256, 333, 1100, 0), (256, 95, 1100, 300),
+                                           (128, 0, 2200, 0), (128, 77, 2200, 0), (128, 77, 2200, 300)])
+def test_fb_one_key_group_lists(ctx, sa, oracle, wo, opts, hd, P, S, window):
+    """One key group with more tiles than workgroups: each workgroup runs a
+    list of pieces (LDS stages used again from piece to piece, cut and whole
+    tiles in one list); with the lists off each piece has a workgroup of its own
+    and the bits are the same. At head_dim 256 (64-row tiles, four waves, three
+    stages) and 128, behind prefixes that end inside a slab and windows that
+    start inside one. Against the oracle without a window, against k_attn_fa
+    with one (1e-5: the two add the same products in other orders, about
+    2^-24 sqrt(slabs) relative)."""
+    from smol_genius_amd.workloads import Prefill
+    n_wg = torch.cuda.get_device_properties(0).multi_processor_count // 16
+    rows = 64 if hd == 256 else 128
+    print("fb one lists", hd, P, S, window, flush=True)
+    assert (S + rows - 1) // rows > n_wg
+    wl = Prefill("t", 16, 16, hd, P, S, 1e5, seed=730 + P + S, in_bf16=False)
+    x = wl.inputs()
+    opts(sa.OPT_PREFILL_KERNEL, 1)
+    opts(sa.OPT_FB_GROUPS, 1)
+    lists, _ = _prefill_with(sa, ctx, wl, x, window)
+    assert ctx.get_option(sa.OPT_FB_WORKGROUPS) <= n_wg
+    opts(sa.OPT_FB_LISTS, -1)
+    pieces, _ = _prefill_with(sa, ctx, wl, x, window)
+    assert ctx.get_option(sa.OPT_FB_WORKGROUPS) > n_wg
+    assert np.array_equal(lists, pieces)
+    if not window:
+        assert_parity(lists, wo.prefill(oracle, wl, x), "fb one lists hd %d P %d S %d" % (hd, P, S))
+    opts(sa.OPT_PREFILL_KERNEL, 2)
+    fa = _prefill_with(sa, ctx, wl, x, window)[0].astype(np.float64)
+    assert np.linalg.norm(lists - fa) <= 1e-5 * np.linalg.norm(fa)
 
 
 @pytest.mark.parametrize("hq,hkv,hd", [(16, 8, 128), (8, 1, 256), (8, 4, 256), (6, 2, 64), (4, 2, 72), (9, 3, 96)])
