@@ -1704,13 +1704,18 @@ extern "C" int smol_attn_prefill_qknorm(smol_attn_ctx *ctx, smol_kv_cache *kv, i
      * transfers, is more than twice as fast as k_attn_fa's (attention and
      * pre-pass, k_attn_fa / widened: 64 tokens of 2 heads a kv head on 8000
      * keys 41 / 43 us, 128 on 8000 55 / 49, 256 on 4096 57 / 43, 500 on 2048
-     * 60 / 44; head_dim 256, 100 tokens on 1000 38 / 31). The staging stays
-     * below 6 bytes x 32768 keys x n_kv x head_dim. */
+     * 60 / 44; head_dim 256, 100 tokens on 1000 38 / 31). The staged prefix
+     * (what the window leaves of it) is bounded, which bounds the workspace it
+     * adds: 6 bytes x 32768 keys x n_kv x head_dim; the call's own rows come on
+     * top. Half that where few rows share it: 100 tokens of 2 heads a kv head
+     * on 16384 keys 88 / 77 us, on 32700 152 / 160. */
     const int pk = ctx->opt[SMOL_OPT_PREFILL_KERNEL];
-    const int seen = pos0 + seq_q - (window > 0 ? std::max(0, pos0 - window + 1) : 0);
+    const int first = window > 0 ? std::max(0, pos0 - window + 1) : 0; /* key that the call can see */
+    const int seen = pos0 + seq_q - first;
     const bool few_keys = seen > 4 * SMOL_SLAB && seen <= 512;
-    const bool widen = seq_q * G > 64 && pk != 2 && (pk == 1 || hd > 128 || seq_q * G > 128 || few_keys) && pos0 <= 32768;
-    const int f0 = (widen ? (window > 0 ? std::max(0, pos0 - window + 1) : 0) : pos0) & ~(SMOL_SLAB - 1);
+    const bool widen = seq_q * G > 64 && pk != 2 && (pk == 1 || hd > 128 || seq_q * G > 128 || few_keys) &&
+                       pos0 - first <= (hd > 128 || seq_q * G > 320 ? 32768 : 16384);
+    const int f0 = (widen ? first : pos0) & ~(SMOL_SLAB - 1);
     const int nf = ((pos0 + seq_q + SMOL_SLAB - 1) & ~(SMOL_SLAB - 1)) - f0;
     pl.pb.push_back({0, seq_q, 0, pos0, 0, seq_q, pos0, f0, nf, 0, slot, 0});
     add_q_blocks(pl, 0, seq_q); /* the Q blocks (the longer ones) dispatched first */

@@ -596,6 +596,30 @@ def test_prefill_form_chosen(sa, ctx, opts, hq, hkv, hd, P, S, window, form):
     assert np.array_equal(auto, want) and not np.array_equal(auto, other)
 
 
+@pytest.mark.parametrize("S,P,window,staged", [
+    (100, 16384, 0, True), (100, 16385, 0, False), (200, 32768, 0, True), (200, 32769, 0, False),
+    (100, 40000, 300, True), (200, 33000, 16500, True), (200, 65600, 32769, True), (200, 65600, 32770, False)])
+def test_prefill_prefix_limit(sa, ctx, oracle, wo, opts, S, P, window, staged):
+    """The prefix that the pre-pass stages is bounded by its own rows (what the
+    window leaves of them), not by the position: on each side of the bounds the
+    bits are those of the route, k_attn_fb over the staged prefix or k_attn_fa
+    over the cache (here 64 pieces a tile, the most), and both meet the oracle
+    (with a window each other, to their sums' order)."""
+    from smol_genius_amd.workloads import Prefill
+    print("prefix limit", S, P, window, flush=True)
+    wl = Prefill("t", 2, 1, 64, P, S, 1e5, seed=740, in_bf16=False)
+    x = wl.inputs()
+    auto, _ = _prefill_with(sa, ctx, wl, x, window)
+    opts(sa.OPT_PREFILL_KERNEL, 2)
+    fa, _ = _prefill_with(sa, ctx, wl, x, window)
+    assert np.array_equal(auto, fa) == (not staged)
+    if not window:
+        want = wo.prefill(oracle, wl, x)
+        assert_parity(auto, want, "prefix limit P %d" % P)
+        assert_parity(fa, want, "prefix limit P %d, k_attn_fa" % P)
+    assert np.linalg.norm(auto - fa) <= 1e-5 * np.linalg.norm(fa)
+
+
 @pytest.mark.parametrize("hq,hkv,hd,P,S,window", [(8, 1, 256, 0, 2500, 512), (8, 1, 256, 2000, 1000, 0)])
 def test_prefill_planning_time(sa, ctx, opts, hq, hkv, hd, P, S, window):
     """Planning a call for k_attn_fb on the host takes no more than three times
