@@ -99,23 +99,47 @@ struct DevBuf {
     size_t cap = 0;
 };
 
-/* grow a device buffer; contents are not kept. The stream is drained first
- * because earlier kernels may still read the old allocation. */
+/* Grow a device buffer; contents are not kept. The stream is drained before
+ * the old allocation goes, because earlier kernels may still read it, and the
+ * new one is made first: an allocation right after a large free waits for the
+ * driver (300 us where it takes 20 otherwise). Only when both do not fit at
+ * once does the old one go first. */
 static int dev_reserve(DevBuf &b, size_t bytes, hipStream_t st, bool zero = false) {
     if (bytes <= b.cap) return 0;
     size_t want = std::max(bytes, b.cap + b.cap / 2);
     want = (want + 4095) & ~(size_t)4095;
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, want);
     if (b.p) {
         HIP_TRY(hipStreamSynchronize(st));
         HIP_TRY(hipFree(b.p));
         b.p = nullptr;
         b.cap = 0;
+        if (e != hipSuccess) {
+            hipGetLastError();
+            e = hipMalloc(&p, want);
+        }
     }
-    HIP_TRY(hipMalloc(&b.p, want));
+    HIP_TRY(e);
+    b.p = p;
     if (zero) HIP_TRY(hipMemsetAsync(b.p, 0, want, st));
     b.cap = want;
     return 0;
 }
+
+/* The arrays a call writes and reads itself, laid out in one allocation
+ * (ctx->work): they are rewritten by every call, in stream order, so nothing
+ * in it outlives a call. One allocation instead of six, and partials only
+ * where tiles are cut: a new context's first prefill of 500 rows behind 2048
+ * written ones spends 80 us on the host, 600 before. */
+struct WorkPlan {
+    size_t bytes = 0;
+    size_t take(size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 1023) & ~(size_t)1023;
+        return at;
+    }
+};
 
 /* ------------------------------------------------ no-alloc decode scratch */
 
@@ -185,9 +209,7 @@ struct smol_attn_ctx {
     int ring_next = 0;
     DevBuf desc;   /* device copy of the descriptor tables */
     std::vector<unsigned char> desc_last; /* host bytes of the last upload to `desc` */
-    DevBuf qs, kf, vtf, part_o, part_ml;
-    DevBuf kf_lo; /* fp16 lo part of the fresh K (precise QK^T) */
-    DevBuf qs32; /* fp32 Q scratch of the decode kernel */
+    DevBuf work;   /* a call's own arrays: Q scratch, staged K and V, partials (WorkPlan) */
     DevBuf out32; /* fp32 result of a call whose output is bf16 */
     DevBuf dec_part; /* k_dec partial slots and flags */
     /* flags, 256 bytes of pinned host memory that kernels write to (only when
@@ -389,8 +411,7 @@ extern "C" int smol_attn_ctx_destroy(smol_attn_ctx *ctx) {
     if (!ctx) return SMOL_ATTN_OK;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
-    DevBuf *bufs[] = {&ctx->desc, &ctx->qs, &ctx->kf, &ctx->kf_lo, &ctx->vtf, &ctx->part_o, &ctx->part_ml,
-                      &ctx->qs32, &ctx->out32, &ctx->dec_part};
+    DevBuf *bufs[] = {&ctx->desc, &ctx->work, &ctx->out32, &ctx->dec_part};
     for (DevBuf *b : bufs)
         if (b->p) hipFree(b->p);
     if (ctx->range_flag) hipHostFree(ctx->range_flag);
@@ -1040,7 +1061,9 @@ struct DecCall {
     std::vector<DecSeq> seqs;
     /* chunk mode: the pre-pass's fresh window and Q scratch */
     int fresh_pos0 = 0, fresh_row0 = 0, fcap = 0;
+    const _Float16 *kf = nullptr, *vtf = nullptr;
     const _Float16 *kf_lo = nullptr; /* the fresh K's lo part (precise QK^T) */
+    const float *qs32 = nullptr;
     long long qs_head_stride = 0;
 };
 
@@ -1234,10 +1257,10 @@ static int run_decode(smol_attn_ctx *ctx, const CallShape &cs, const DecCall &dc
         }
         dp.q_norm = cs.q_norm; dp.k_norm = cs.k_norm; dp.norm_eps = cs.norm_eps;
     } else {
-        dp.kf = (const _Float16 *)ctx->kf.p; dp.vtf = (const _Float16 *)ctx->vtf.p; dp.fcap = dc.fcap;
+        dp.kf = dc.kf; dp.vtf = dc.vtf; dp.fcap = dc.fcap;
         dp.kf_lo = dc.kf_lo;
         dp.fresh_pos0 = dc.fresh_pos0; dp.fresh_row0 = dc.fresh_row0;
-        dp.qs32 = (const float *)ctx->qs32.p; dp.qs_head_stride = dc.qs_head_stride;
+        dp.qs32 = dc.qs32; dp.qs_head_stride = dc.qs_head_stride;
     }
     dp.qscale = (float)(cs.scale * LOG2E_D);
     dp.out = cs.out; dp.Hq = cs.Hq; dp.Hkv = cs.Hkv; dp.G = G;
@@ -1463,21 +1486,22 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     int rc;
     const size_t fcap = (size_t)std::max(pl.fresh_rows, SMOL_SLAB);
     const size_t qs_elems = (size_t)cs.Hkv * std::max(pl.q_rows, 1) * hdp;
-    if (cs.dec) {
-        if ((rc = dev_reserve(ctx->qs32, qs_elems * 4, ctx->stream))) return rc;
-    } else {
-        if ((rc = dev_reserve(ctx->qs, qs_elems * 2 * (precise ? 2 : 1), ctx->stream))) return rc;
-    }
-    if ((rc = dev_reserve(ctx->kf, (size_t)cs.Hkv * fcap * hd * 2, ctx->stream))) return rc;
-    if (precise && (rc = dev_reserve(ctx->kf_lo, (size_t)cs.Hkv * fcap * hd * 2, ctx->stream))) return rc;
-    _Float16 *const qs_lo = precise && !cs.dec ? (_Float16 *)ctx->qs.p + qs_elems : nullptr;
-    _Float16 *const kf_lo = precise ? (_Float16 *)ctx->kf_lo.p : nullptr;
-    if ((rc = dev_reserve(ctx->vtf, (size_t)cs.Hkv * fcap * hd * 2, ctx->stream))) return rc;
     const size_t n_items = pl.items.size();
-    if (fa) {
-        if ((rc = dev_reserve(ctx->part_o, std::max<size_t>(1, n_items) * cs.Hkv * rows_per * hd * 4, ctx->stream))) return rc;
-        if ((rc = dev_reserve(ctx->part_ml, std::max<size_t>(1, n_items) * cs.Hkv * rows_per * 2 * 4, ctx->stream))) return rc;
-    }
+    bool split = false; /* k_attn_fa and k_attn_fb write partials of cut tiles only */
+    for (const SkItem &it : pl.items) split |= fa && it.n_split > 1;
+    WorkPlan wk;
+    const size_t kv_bytes = (size_t)cs.Hkv * fcap * hd * 2;
+    const size_t o_qs = wk.take(qs_elems * (cs.dec ? 4 : precise ? 4 : 2));
+    const size_t o_kf = wk.take(kv_bytes), o_kf_lo = wk.take(precise ? kv_bytes : 0), o_vtf = wk.take(kv_bytes);
+    const size_t o_po = wk.take(split ? n_items * cs.Hkv * rows_per * hd * 4 : 0);
+    const size_t o_ml = wk.take(split ? n_items * cs.Hkv * rows_per * 2 * 4 : 0);
+    if ((rc = dev_reserve(ctx->work, wk.bytes, ctx->stream))) return rc;
+    unsigned char *const work = (unsigned char *)ctx->work.p;
+    _Float16 *const qs = cs.dec ? nullptr : (_Float16 *)(work + o_qs);
+    float *const qs32 = cs.dec ? (float *)(work + o_qs) : nullptr;
+    _Float16 *const qs_lo = precise && !cs.dec ? qs + qs_elems : nullptr;
+    _Float16 *const kf = (_Float16 *)(work + o_kf), *const vtf = (_Float16 *)(work + o_vtf);
+    _Float16 *const kf_lo = precise ? (_Float16 *)(work + o_kf_lo) : nullptr;
 
     /* k_attn_fb with more tiles than compute units: one workgroup per unit
      * and kv head runs a list of tiles, assigned longest first to the least
@@ -1553,13 +1577,13 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     pp.rope_k = cs.rope_k;
     pp.qscale = (float)(cs.scale * LOG2E_D);
     pp.Hq = cs.Hq; pp.Hkv = cs.Hkv; pp.G = G; pp.hd = hd; pp.hdp = hdp;
-    pp.qs = (_Float16 *)ctx->qs.p;
+    pp.qs = qs;
     pp.qs_head_stride = (long long)std::max(pl.q_rows, 1) * hdp;
     pp.kc = kc; pp.vtc = vtc; pp.c_slot_stride = slot_stride; pp.cap = cap;
-    pp.kf = (_Float16 *)ctx->kf.p; pp.vtf = (_Float16 *)ctx->vtf.p; pp.fcap = (int)fcap;
+    pp.kf = kf; pp.vtf = vtf; pp.fcap = (int)fcap;
     pp.qs_lo = qs_lo; pp.kf_lo = kf_lo;
     pp.stage = cs.dec ? SMOL_STAGE_QF32 : SMOL_STAGE_F16;
-    if (cs.dec) pp.qs32 = (float *)ctx->qs32.p;
+    if (cs.dec) pp.qs32 = qs32;
     pp.blocks = (const PrepBlockB *)(dd + o_pblk);
     pp.q_norm = cs.q_norm; pp.k_norm = cs.k_norm; pp.norm_eps = cs.norm_eps;
     pp.range_flag = ctx->range_flag;
@@ -1580,17 +1604,20 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
         dc.fresh_pos0 = b.fresh_pos0;
         dc.fresh_row0 = b.fresh_row0;
         dc.fcap = (int)fcap;
+        dc.kf = kf;
+        dc.vtf = vtf;
         dc.kf_lo = kf_lo;
+        dc.qs32 = qs32;
         dc.qs_head_stride = pp.qs_head_stride;
         return run_decode(ctx, cs, dc);
     }
 
     SkParams sp;
     memset(&sp, 0, sizeof(sp));
-    sp.qs = (const _Float16 *)ctx->qs.p;
+    sp.qs = qs;
     sp.qs_head_stride = pp.qs_head_stride;
     sp.kc = kc; sp.vtc = vtc; sp.c_slot_stride = slot_stride; sp.cap = cap;
-    sp.kf = (const _Float16 *)ctx->kf.p; sp.vtf = (const _Float16 *)ctx->vtf.p; sp.fcap = (int)fcap;
+    sp.kf = kf; sp.vtf = vtf; sp.fcap = (int)fcap;
     sp.qs_lo = qs_lo; sp.kf_lo = kf_lo;
     sp.out = cs.out;
     sp.Hq = cs.Hq; sp.Hkv = cs.Hkv; sp.G = G;
@@ -1598,8 +1625,8 @@ static int run_plan(smol_attn_ctx *ctx, Plan &pl, const CallShape &cs) {
     sp.cap2 = cs.cap > 0.0f ? (float)(cs.cap * LOG2E_D) : 0.0f;
     sp.range_flag = ctx->range_flag;
     sp.items = (const SkItemB *)(dd + o_it);
-    sp.part_o = (float *)ctx->part_o.p;
-    sp.part_ml = (float *)ctx->part_ml.p;
+    sp.part_o = (float *)(work + o_po);
+    sp.part_ml = (float *)(work + o_ml);
     if (fb) {
         sp.fb_items = (const FbItem *)(dd + o_sc);
         sp.n_wg = fb_wg;
@@ -1954,8 +1981,11 @@ extern "C" int smol_kv_cache_write(smol_kv_cache *kv, int layer, int slot, int p
     pl.fresh_rows = nf;
     const int hd = kv->hd;
     const size_t fcap = (size_t)nf;
-    if ((rc = dev_reserve(ctx->kf, (size_t)kv->n_kv * fcap * hd * 2, ctx->stream))) return rc;
-    if ((rc = dev_reserve(ctx->vtf, (size_t)kv->n_kv * fcap * hd * 2, ctx->stream))) return rc;
+    WorkPlan wk;
+    const size_t o_kf = wk.take((size_t)kv->n_kv * fcap * hd * 2), o_vtf = wk.take((size_t)kv->n_kv * fcap * hd * 2);
+    if ((rc = dev_reserve(ctx->work, wk.bytes, ctx->stream))) return rc;
+    _Float16 *const kf = (_Float16 *)((unsigned char *)ctx->work.p + o_kf);
+    _Float16 *const vtf = (_Float16 *)((unsigned char *)ctx->work.p + o_vtf);
     const std::vector<PrepBlockB> pbr = prep_records(pl, false, kv->n_kv, 3 * ctx->cu_count);
     if ((rc = upload_desc(ctx, pbr.data(), pbr.size() * sizeof(PrepBlockB)))) return rc;
     PrepParams pp;
@@ -1968,7 +1998,7 @@ extern "C" int smol_kv_cache_write(smol_kv_cache *kv, int layer, int slot, int p
     pp.vtc = kv->vt + (size_t)layer * kv_layer_elems(kv);
     pp.c_slot_stride = (long long)kv_slot_elems(kv);
     pp.cap = kv->cap;
-    pp.kf = (_Float16 *)ctx->kf.p; pp.vtf = (_Float16 *)ctx->vtf.p; pp.fcap = (int)fcap;
+    pp.kf = kf; pp.vtf = vtf; pp.fcap = (int)fcap;
     pp.blocks = (const PrepBlockB *)ctx->desc.p;
     rc = smol_launch_prep(&pp, (int)pbr.size(), ctx->stream, nullptr, nullptr);
     if (!on_device) {

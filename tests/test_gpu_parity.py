@@ -636,6 +636,42 @@ def test_prefill_planning_time(sa, ctx, opts, hq, hkv, hd, P, S, window):
     assert fb <= 3 * fa
 
 
+def test_first_prefill_of_a_context(sa):
+    """The first prefill behind written rows on a new context: growing the
+    workspace for the staged prefix may cost the host no more than four times
+    what k_attn_fa's small one does (it was ten times: an allocation right
+    after a free, and six of them)."""
+    from smol_genius_amd.workloads import Prefill
+    wl = Prefill("t", 16, 8, 128, 2048, 500, 1e6, seed=760, in_bf16=False)
+    x = wl.inputs()
+    args = [dev(x[n]) for n in ("q", "k", "v")]
+    rows = [dev(x[n], True) for n in ("cache_k", "cache_v")]
+
+    def first_call(kernel):
+        us = []
+        for _ in range(7):
+            c = sa.Context(0)
+            c.set_option(sa.OPT_PREFILL_KERNEL, kernel)
+            kv = sa.KVCache(c, 1, 1, wl.Hkv, wl.hd, wl.pos0 + wl.seq_q)
+            kv.write(0, 0, 0, *rows)
+            rope = sa.RopeTable(c, wl.hd, wl.theta, 0, wl.pos0 + wl.seq_q)
+            call = sa.prefill_call(c, kv, 0, 0, rope, wl.pos0, *args, wl.Hq, wl.scale)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            call()
+            us.append(1e6 * (time.perf_counter() - t))
+            torch.cuda.synchronize()
+            kv.close()
+            rope.close()
+            c.close()
+        return float(np.median(us[2:]))
+
+    print("first prefill", flush=True)
+    fa, fb = first_call(2), first_call(0)
+    print("host us: k_attn_fa %.0f, staged prefix %.0f" % (fa, fb), flush=True)
+    assert fb <= 4 * fa
+
+
 @pytest.mark.parametrize("window,cap", [(16, 0.0), (0, 2.0), (1, 0.0), (40, 1.5), (1, 3.0)])
 def test_decode_window_softcap(ctx, sa, oracle, wo, window, cap):
     """Sliding window and softcap on decode (the new key is scored apart
@@ -791,10 +827,13 @@ def test_fresh_context_long_prefill(sa, oracle, wo):
         c.close()
 
 
-def test_long_prefix_chunk(ctx, sa, oracle, wo):
-    """A 64-token chunk on a 16384-token cache (k_attn_fa, key ranges split across workgroups)."""
+@pytest.mark.parametrize("kernel", [2, 0], ids=["k_attn_fa", "default"])
+def test_long_prefix_chunk(ctx, sa, oracle, wo, opts, kernel):
+    """A 64-token chunk on a 16384-token cache: k_attn_fa, key ranges split
+    across workgroups, and the default, k_attn_fb over the staged prefix."""
     from smol_genius_amd.workloads import Prefill
-    print("chunk 64 on 16384", flush=True)
+    print("chunk 64 on 16384", kernel, flush=True)
+    opts(sa.OPT_PREFILL_KERNEL, kernel)
     wl = Prefill("t", 8, 2, 128, 16384, 64, 1e6, seed=121)
     x = wl.inputs()
     kv = sa.KVCache(ctx, 1, 1, 2, 128, 16384 + 64)
