@@ -347,25 +347,22 @@ static int upload_desc(smol_attn_ctx *ctx, const void *host, size_t bytes) {
  * workgroup ran where workgroup b % n_xcc ran, not on XCD b % n_xcc: that
  * form failed on three streams of four and left their decode calls without
  * splits (Qwen3-0.6B sizes, 1025 keys: 19.8 us a layer, 12.3 with them). A
- * probe grid records each workgroup's XCC id; when one differs from its
+ * probe grid records each workgroup's XCC id (in `ids`, pinned host memory:
+ * the context's flags, which it needs anyway; an allocation and a copy of the
+ * probe's own made creation 66 us instead of XX); when one differs from its
  * class, k_dec keeps every group in one workgroup. */
-static int check_xcd_dispatch(smol_attn_ctx *c) {
-    int nx = 0;
-    if (hipDeviceGetAttribute(&nx, hipDeviceAttributeNumberOfXccs, c->device) != hipSuccess || nx <= 0) nx = 1;
-    c->n_xcc = nx;
+#define XCD_PROBES 64 /* workgroups a class */
+static int check_xcd_dispatch(smol_attn_ctx *c, unsigned *ids) {
     c->xcd_ok = true;
-    if (nx == 1) return 0;
-    const int n = 64 * nx;
-    unsigned *d = nullptr;
-    HIP_TRY(hipMalloc(&d, n * sizeof(unsigned)));
-    std::vector<unsigned> h(n, 0xFFFFFFFFu);
-    int rc = smol_launch_xcc_probe(d, n, c->stream);
-    hipError_t e = rc ? hipErrorLaunchFailure : hipMemcpyAsync(h.data(), d, n * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    hipFree(d);
+    if (c->n_xcc == 1) return 0;
+    const int n = XCD_PROBES * c->n_xcc;
+    memset(ids, 0xFF, n * sizeof(unsigned));
+    const int rc = smol_launch_xcc_probe(ids, n, c->stream);
+    const hipError_t e = rc ? hipErrorLaunchFailure : hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return fail(SMOL_ATTN_ERR_DEVICE, "XCD probe: %s", hipGetErrorString(e));
+    const volatile unsigned *h = ids;
     for (int b = 0; b < n; b++)
-        if (h[b] == 0xFFFFFFFFu || h[b] != h[b % nx]) c->xcd_ok = false;
+        if (h[b] == 0xFFFFFFFFu || h[b] != h[b % c->n_xcc]) c->xcd_ok = false;
     return 0;
 }
 
@@ -389,15 +386,17 @@ extern "C" int smol_attn_ctx_create(int device, void *stream, smol_attn_ctx **ou
         delete c;
         return fail(SMOL_ATTN_ERR_DEVICE, "context: %s", hipGetErrorString(e));
     }
+    int nx = 0;
+    if (hipDeviceGetAttribute(&nx, hipDeviceAttributeNumberOfXccs, device) == hipSuccess && nx > 0) c->n_xcc = nx;
     int rc = scratch_setup(device);
-    if (!rc) rc = check_xcd_dispatch(c);
     if (!rc) {
-        if (hipHostMalloc((void **)&c->range_flag, 4 * SMOL_FLAG_WORDS,
-                          hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) == hipSuccess)
-            memset(c->range_flag, 0, 4 * SMOL_FLAG_WORDS);
-        else
-            rc = fail(SMOL_ATTN_ERR_NOMEM, "range flag: %s", hipGetErrorString(hipGetLastError()));
+        const size_t bytes = std::max<size_t>(4 * SMOL_FLAG_WORDS, sizeof(unsigned) * XCD_PROBES * c->n_xcc);
+        if (hipHostMalloc((void **)&c->range_flag, bytes,
+                          hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess)
+            rc = fail(SMOL_ATTN_ERR_NOMEM, "context flags: %s", hipGetErrorString(hipGetLastError()));
     }
+    if (!rc) rc = check_xcd_dispatch(c, (unsigned *)c->range_flag);
+    if (!rc) memset(c->range_flag, 0, 4 * SMOL_FLAG_WORDS);
     if (rc) {
         if (c->range_flag) hipHostFree(c->range_flag);
         delete c;
