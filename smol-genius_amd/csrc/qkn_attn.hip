@@ -258,7 +258,8 @@ int run_layer(Binding *b, int layer, int pos, int n, float *x, const smol_qkn_la
     int rc;
     if ((rc = reserve(b, b->lq, (size_t)n * q_dim * 4)) || (rc = reserve(b, b->lk, (size_t)n * kv_dim * 4)) ||
         (rc = reserve(b, b->lv, (size_t)n * kv_dim * 4)) || (rc = reserve(b, b->la, (size_t)n * q_dim * 4)) ||
-        (rc = reserve(b, b->lp, (size_t)n * dim * 4)) || (rc = reserve(b, b->lg, (size_t)n * inter * 4)))
+        (rc = reserve(b, b->lp, (size_t)n * dim * 4)) || (rc = reserve(b, b->lg, (size_t)n * inter * 4)) ||
+        (!decode && (rc = reserve(b, b->ly, (size_t)n * dim * 4))))
         return rc;
     float *q = (float *)b->lq.p, *k = (float *)b->lk.p, *v = (float *)b->lv.p;
     float *attn = (float *)b->la.p, *p = (float *)b->lp.p, *g = (float *)b->lg.p;
@@ -269,7 +270,7 @@ int run_layer(Binding *b, int layer, int pos, int n, float *x, const smol_qkn_la
     if ((rc = run_block(b, layer, pos, n, q, k, v, attn, decode, false))) return rc;
     float *y = x; /* x + attention */
     if (!decode) {
-        if ((rc = reserve(b, b->ly, (size_t)n * dim * 4)) || (rc = smol_internal_mark(ctx))) return rc;
+        if ((rc = smol_internal_mark(ctx))) return rc;
         y = (float *)b->ly.p;
     }
     smol_linear_ops ops{};
@@ -324,7 +325,8 @@ int run_layer_bf16(Binding *b, int layer, int pos, int n, uint16_t *x, const smo
     if ((rc = reserve(b, b->lq, (size_t)n * q_dim * 2)) || (rc = reserve(b, b->lk, (size_t)n * kv_dim * 2)) ||
         (rc = reserve(b, b->lv, (size_t)n * kv_dim * 2)) || (rc = reserve(b, b->la, (size_t)n * q_dim * 2)) ||
         (rc = reserve(b, b->lp, (size_t)n * dim * 2)) || (rc = reserve(b, b->lg, (size_t)n * 2 * inter * 2)) ||
-        (rc = reserve(b, b->lx, (size_t)n * dim * 2)) || (rc = reserve(b, b->lh, (size_t)n * inter * 2)))
+        (rc = reserve(b, b->lx, (size_t)n * dim * 2)) || (rc = reserve(b, b->lh, (size_t)n * inter * 2)) ||
+        (!decode && (rc = reserve(b, b->ly, (size_t)n * dim * 2))))
         return rc;
     uint16_t *q = (uint16_t *)b->lq.p, *k = (uint16_t *)b->lk.p, *v = (uint16_t *)b->lv.p;
     uint16_t *attn = (uint16_t *)b->la.p, *p = (uint16_t *)b->lp.p, *gu = (uint16_t *)b->lg.p;
@@ -368,10 +370,7 @@ int run_layer_bf16(Binding *b, int layer, int pos, int n, uint16_t *x, const smo
         }
     }
     uint16_t *y = x; /* x + attention */
-    if (!decode) {
-        if ((rc = reserve(b, b->ly, (size_t)n * dim * 2))) return rc;
-        y = (uint16_t *)b->ly.p;
-    }
+    if (!decode) y = (uint16_t *)b->ly.p;
     if (w->pre_ffn_norm)
         rc = smol_internal_bf16_add_norm(ctx, x, y, p, w->post_attn_norm, w->pre_ffn_norm, xn, n, dim, c.eps);
     else
