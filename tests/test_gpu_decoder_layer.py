@@ -343,3 +343,61 @@ def test_layer_range_error_leaves_x(sa, bf16, rows, gemma):
         assert torch.equal(call(y, good), want) and not torch.equal(want, x.cpu())
     finally:
         blk.close()
+
+
+@pytest.mark.parametrize("rows", [5, 40, 130, 333])
+@pytest.mark.parametrize("dim,inter,gemma", [(256, 384, False), (256, 390, True), (1024, 3072, False)])
+def test_bf16_layer_is_its_parts(sa, rows, dim, inter, gemma):
+    """A bf16 prefill layer (GeGLU in the gate_up launch, the sum with the
+    attention kept apart) has the bits of its parts called one by one: norm,
+    Q/K/V, the attention block, projections, the residual adds with their norms,
+    and gate_up and GeGLU as two launches. 390 pairs leave half a tile."""
+    H, Hkv, hd = 4, 2, 64
+    print("bf16 layer parts", rows, dim, inter, gemma, flush=True)
+    ctx = sa.Context(0)
+    owners = [ctypes.create_string_buffer(256) for _ in range(2)]
+    blks = [sa.QknAttn(o, n_layers=1, n_heads=H, n_kv_heads=Hkv, head_dim=hd, eps=1e-6, rope_theta=1e6,
+                       rope_local_theta=0.0, rope_type=0, sliding_window=0, attn_logit_softcap=0.0, bf16=1,
+                       on_device=1, device=0, max_seq=512) for o in owners]
+
+    def d(a):
+        a = np.ascontiguousarray(a)
+        return torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).cuda()
+
+    def bf(t):
+        return t.view(torch.bfloat16)
+
+    try:
+        qn, kn = (1.0 + 0.1 * synth.normal(920 + i, (hd,)).astype(np.float32) for i in range(2))
+        for b in blks:
+            b.set_layer(0, 0, qn, kn)
+        w = dict(input_norm=d(_norm_w(921, dim)), wq=d(_proj(922, H * hd, dim)), wk=d(_proj(923, Hkv * hd, dim)),
+                 wv=d(_proj(924, Hkv * hd, dim)), wo=d(_proj(925, dim, H * hd)), post_attn_norm=d(_norm_w(926, dim)),
+                 pre_ffn_norm=d(_norm_w(927, dim)) if gemma else None,
+                 post_ffn_norm=d(_norm_w(928, dim)) if gemma else None, gate_up=d(_proj(929, 2 * inter, dim)),
+                 down=d(_proj(930, dim, inter)))
+        x = bf(d(synth.f32_to_bf16_bits(synth.normal(931, (rows, dim)))))
+        torch.cuda.synchronize()
+        got = blks[0].layer_prefill_bf16(0, 0, x.clone(), sa.QknLayerWeights(**w), dim, inter)
+        blks[0].synchronize()
+
+        n = sa.bf16_rms_norm(ctx, x, w["input_norm"], 1e-6)
+        q, k, v = sa.linear_qkv(ctx, bf(n), w["wq"], w["wk"], w["wv"], out_bf16=True)
+        ctx.synchronize()
+        attn = blks[1].prefill(0, 0, bf(q), bf(k), bf(v))
+        blks[1].synchronize()
+        p = sa.linear(ctx, bf(attn), w["wo"], out_bf16=True)
+        y = x.clone()
+        if gemma:
+            n = sa.bf16_add_norm(ctx, y, bf(p), w["post_attn_norm"], w["pre_ffn_norm"])
+        else:
+            n = sa.bf16_add_norm(ctx, y, bf(p), None, w["post_attn_norm"])
+        g = sa.bf16_geglu(ctx, sa.linear(ctx, bf(n), w["gate_up"], out_bf16=True))
+        f = sa.linear(ctx, bf(g), w["down"], out_bf16=True)
+        sa.bf16_add_norm(ctx, y, bf(f), w["post_ffn_norm"])
+        ctx.synchronize()
+        assert torch.equal(got.view(torch.int16), y.view(torch.int16))
+    finally:
+        for b in blks:
+            b.close()
+        ctx.close()
