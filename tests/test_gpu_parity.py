@@ -515,6 +515,26 @@ def test_fb_one_key_group_lists(ctx, sa, oracle, wo, opts, hd, P, S, window):
     opts(sa.OPT_PREFILL_KERNEL, 2)
     fa = _prefill_with(sa, ctx, wl, x, window)[0].astype(np.float64)
     assert np.linalg.norm(lists - fa) <= 1e-5 * np.linalg.norm(fa)
+    if not window:  # single fp16 operands: a build of its own
+        opts(sa.OPT_QK_FP16, 1)
+        opts(sa.OPT_PREFILL_KERNEL, 1)
+        opts(sa.OPT_FB_LISTS, 0)
+        lists, _ = _prefill_with(sa, ctx, wl, x, window)
+        assert_parity(lists, wo.prefill(oracle, wl, x), "fb one lists fp16 hd %d P %d S %d" % (hd, P, S))
+
+
+@pytest.mark.parametrize("ws", [[0, 100, 700, 750, 1500], [3, 1103]])
+def test_bidirectional_head_dim_256(ctx, sa, oracle, ws):
+    """Windows at head_dim 256 (k_attn_fb's one key group over several batches,
+    cut and whole tiles): ragged windows and a long one, fp32 rows."""
+    H, hd, seq = 4, 256, ws[-1]
+    print("bidirectional 256", ws, flush=True)
+    Q, K, V = (synth.normal(770 + i, (seq, H * hd)) for i in range(3))
+    sc = 1.0 / np.sqrt(hd)
+    out = torch.zeros((seq, H * hd), dtype=torch.float32, device="cuda")
+    got = sa.bidirectional(ctx, dev(Q), dev(K), dev(V), seq, H, hd, sc, ws, out=out).cpu().numpy()
+    ctx.synchronize()
+    assert_parity(got[ws[0]:], oracle.bidirectional_attention(Q, K, V, seq, H, hd, sc, ws)[ws[0]:], "bidir 256 %s" % ws)
 
 
 @pytest.mark.parametrize("hq,hkv,hd", [(16, 8, 128), (8, 1, 256), (8, 4, 256), (6, 2, 64), (4, 2, 72), (9, 3, 96)])
