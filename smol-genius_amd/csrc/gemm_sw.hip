@@ -23,11 +23,13 @@
  * 2048, 15.7 us.)
  *
  * Measured, weights not in L2, k_gemm's 64 x 64 tile / K split over the waves
- * / this kernel (us): 26 fp32 rows, 6144 -> 2048 49.5 / 12.8 / 12.9 (25 MB of
- * weights: 2 TB/s); 2048 -> 2048 18.1 / 7.0 / 6.8; 2048 -> 12288 with the norm
- * and SwiGLU 22.9 / 15.0 / 15.0 (50 MB: 3.4 TB/s); 333 bf16 rows, 3072 -> 1024
- * 24.4 / 13.0 / 12.8; 5 bf16 rows, 6144 -> 2048 44 / 9.0 / 10.9; 333 bf16 rows,
- * 1024 -> 6144 20.5 / - / 18.0. The host chooses by a fitted cost of each tile
+ * / this kernel (us): 26 fp32 rows, 6144 -> 2048 49.5 / 12.5 / 13.2 (25 MB of
+ * weights: 1.9 TB/s); 2048 -> 2048 18.1 / 6.2 / 6.5; 2048 -> 12288 with the norm
+ * and SwiGLU 22.9 / 15.1 / 14.6 (50 MB: 3.4 TB/s); 333 bf16 rows, 3072 -> 1024
+ * 24.4 / 12.6 / 12.8; 5 bf16 rows, 6144 -> 2048 44 / 9.4 / 11.2. Chunks
+ * swizzled by four row bits where a row has 16 or more: 15% of the LDS cycles
+ * were conflicts with three, and those tiles took 2 to 12% longer. The host
+ * chooses by a fitted cost of each tile
  * (gemm_cfg, linear.hip); without k_gemm's own 64 x 64 tile that choice is
  * 0.03% worse on average over 484 products, so that tile is gone.
  */
@@ -41,6 +43,7 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
     constexpr int CPR = KC / 8;   /* 16-byte bf16 chunks of a row of a slab */
     constexpr int ROWB = KC * 2;  /* bytes of an LDS row */
     constexpr int RS = TPB / CPR; /* rows between two chunks of a staging thread */
+    constexpr int SWZ = CPR < 16 ? 7 : 15; /* row bits that swizzle a chunk: a fragment's rows then span every bank */
     /* a stage: W, x (hi), x lo, and with the norm x as loaded (the first four
      * values of each chunk, then the last four) */
     constexpr int XH = BN * ROWB, XLO = XH + BM * ROWB, XR = XLO + (XBF ? 0 : BM * ROWB);
@@ -48,7 +51,7 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
     constexpr int WL = BN * CPR / TPB, XL = BM * CPR / TPB; /* chunks a thread stages of W and x */
     static_assert(2 * STAGE <= 160 * 1024, "LDS");
     static_assert(WL * TPB == BN * CPR && XL * TPB == BM * CPR, "staging shape");
-    static_assert(RS % 8 == 0, "every row of a thread has one swizzle");
+    static_assert(RS % (SWZ + 1) == 0, "every row of a thread has one swizzle");
     static_assert(KS % 2 == 0, "fragments are read two steps at a time");
     static_assert(!(XBF && NORM), "the norm takes an fp32 x");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * STAGE];
@@ -81,9 +84,7 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
         for (int e = 0; e < WL; e++) w_off[e] = (unsigned)(((lr + RS * e) * K + 8 * lq) * 2);
 #pragma unroll
         for (int e = 0; e < XL; e++) x_off[e] = (unsigned)(((lr + RS * e) * K + 8 * lq) * xes);
-        /* 16-byte chunks XOR-swizzled by the row's low 3 bits: the fragment
-         * reads of eight consecutive lanes hit distinct banks */
-        const unsigned pos = (unsigned)(lr * ROWB + ((lq ^ (lr & 7)) << 4));
+        const unsigned pos = (unsigned)(lr * ROWB + ((lq ^ (lr & SWZ)) << 4));
 
         struct Raw {
             uint4 w[WL], x[XL][XP], g[NORM ? 2 : 1];
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
 
     /* lane (c, j): chunk 4 ks + j of a row, step ks of the slab */
     auto frag = [&](const unsigned char *base, int row, int ks) __attribute__((always_inline)) {
-        return *reinterpret_cast<const uint4 *>(base + row * ROWB + (((4 * ks + j) ^ (row & 7)) << 4));
+        return *reinterpret_cast<const uint4 *>(base + row * ROWB + (((4 * ks + j) ^ (row & SWZ)) << 4));
     };
     if (NORM && wave >= SW + MW) {
         const int row = 16 * (wave - SW - MW) + c;

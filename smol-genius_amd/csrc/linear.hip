@@ -738,22 +738,22 @@ int run_gemv_rows(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const v
  * K in thousands. The constants are fitted (least squares of the relative
  * error) to the measured times of every configuration at 5 to 2048 rows, 640 to
  * 12288 outputs and K = 640 to 6144, weights not in L2, for a plain fp32 x, one
- * with the norm and a bf16 x; over those 484 products the choice is within 0.7%
+ * with the norm and a bf16 x; over those 484 products the choice is within 0.8%
  * of the best configuration on average, 26% at worst (1300 bf16 rows, 6144 ->
- * 2048: 83.9 us against 66.6). The bits are the same in every one of them.
+ * 2048: 83.2 us against 65.8). The bits are the same in every one of them.
  * Where the lines fall (rows up to which a k_gemm_sw tile is chosen): N = 1024,
  * K = 1024 to 3072: 2048 and more; N = 6144, K = 1024: 320; N = 12288, K = 2048
  * with the norm: 128. */
 int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, bool norm, int seg_align = 0) {
     static const float cost[GEMM_CFGS][3][4] = {
-        {{0.0f, 7.89f, 25.9f, 0.0737f}, {0.0f, 9.66f, 27.5f, 0.186f}, {0.0f, 6.91f, 17.1f, 0.0f}},
-        {{0.0f, 3.59f, 14.9f, 0.137f}, {0.0f, 5.56f, 17.9f, 0.0342f}, {0.0f, 5.43f, 10.5f, 0.0f}},
-        {{4.68f, 0.0f, 5.37f, 0.0745f}, {2.13f, 3.21f, 7.37f, 0.00928f}, {3.83f, 1.26f, 3.52f, 0.00656f}},
-        {{0.0f, 4.63f, 8.72f, 0.0996f}, {0.0f, 6.23f, 10.1f, 0.0325f}, {0.573f, 5.81f, 5.87f, 0.0f}},
-        {{2.05f, 2.25f, 4.12f, 0.0f}, {1.99f, 3.19f, 4.88f, 0.00881f}, {3.73f, 1.04f, 2.65f, 0.0192f}},
-        {{1.84f, 2.19f, 2.91f, 0.0f}, {2.72f, 2.11f, 4.03f, 0.0125f}, {3.77f, 0.865f, 1.62f, 0.0166f}},
-        {{2.26f, 1.75f, 1.86f, 0.00487f}, {2.28f, 2.98f, 2.09f, 0.0f}, {3.46f, 0.716f, 1.07f, 0.0339f}},
-        {{3.32f, 0.963f, 1.29f, 0.0105f}, {2.53f, 2.61f, 1.68f, 0.0104f}, {3.11f, 0.899f, 0.758f, 0.0319f}},
+        {{0.0f, 7.81f, 25.9f, 0.0444f}, {0.0f, 9.65f, 27.7f, 0.162f}, {0.0f, 6.44f, 17.1f, 0.0f}},
+        {{0.0f, 3.45f, 14.9f, 0.145f}, {0.0f, 5.34f, 17.8f, 0.0385f}, {0.0f, 5.27f, 10.5f, 0.00143f}},
+        {{4.29f, 0.0f, 5.44f, 0.0669f}, {2.23f, 2.86f, 7.52f, 0.0f}, {3.85f, 1.18f, 3.48f, 0.0108f}},
+        {{0.0f, 3.99f, 8.93f, 0.0779f}, {0.0f, 5.94f, 10.2f, 0.0257f}, {0.871f, 5.58f, 5.78f, 0.0f}},
+        {{1.87f, 2.09f, 3.61f, 0.0f}, {1.83f, 3.1f, 4.32f, 0.0104f}, {3.74f, 1.14f, 2.26f, 0.0214f}},
+        {{1.61f, 1.98f, 2.71f, 0.0f}, {2.59f, 2.01f, 3.61f, 0.0f}, {3.41f, 0.987f, 1.4f, 0.0243f}},
+        {{2.17f, 1.68f, 1.76f, 0.0f}, {2.04f, 3.01f, 1.91f, 0.0117f}, {3.51f, 0.751f, 1.01f, 0.0302f}},
+        {{3.14f, 0.951f, 1.27f, 0.0261f}, {2.47f, 2.59f, 1.59f, 0.00759f}, {3.33f, 0.897f, 0.732f, 0.027f}},
     };
     const int forced = smol_internal_ctx_option(ctx, SMOL_OPT_GEMM_TILE);
     if (forced >= 1 && forced <= GEMM_CFGS) {
