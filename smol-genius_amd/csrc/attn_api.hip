@@ -97,33 +97,38 @@ static bool hd_supported(int hd) {
 struct DevBuf {
     void *p = nullptr;
     size_t cap = 0;
+    std::vector<void *> old; /* smaller allocations that kernels may still read */
 };
 
-/* Grow a device buffer; contents are not kept. The stream is drained before
- * the old allocation goes, because earlier kernels may still read it, and the
- * new one is made first: an allocation right after a large free waits for the
- * driver (300 us where it takes 20 otherwise). Only when both do not fit at
- * once does the old one go first. */
+static void dev_free(DevBuf &b) {
+    if (b.p) hipFree(b.p);
+    for (void *p : b.old) hipFree(p);
+    b = DevBuf();
+}
+
+/* Grow a device buffer; contents are not kept. The allocations before it stay
+ * until the buffer goes: earlier kernels may still read them, so freeing one
+ * drains the stream, and an allocation after a large free waits for the driver
+ * (300 us where it takes 20 otherwise). Capacities double, so what stays is
+ * less than the buffer itself; when the device has no room it goes first. */
 static int dev_reserve(DevBuf &b, size_t bytes, hipStream_t st, bool zero = false) {
     if (bytes <= b.cap) return 0;
-    size_t want = std::max(bytes, b.cap + b.cap / 2);
+    size_t want = std::max(bytes, 2 * b.cap);
     want = (want + 4095) & ~(size_t)4095;
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, want);
-    if (b.p) {
+    if (e != hipSuccess) {
+        hipGetLastError();
         HIP_TRY(hipStreamSynchronize(st));
-        HIP_TRY(hipFree(b.p));
-        b.p = nullptr;
-        b.cap = 0;
-        if (e != hipSuccess) {
-            hipGetLastError();
-            e = hipMalloc(&p, want);
-        }
+        dev_free(b);
+        want = (bytes + 4095) & ~(size_t)4095;
+        e = hipMalloc(&p, want);
     }
     HIP_TRY(e);
+    if (b.p) b.old.push_back(b.p);
     b.p = p;
-    if (zero) HIP_TRY(hipMemsetAsync(b.p, 0, want, st));
     b.cap = want;
+    if (zero) HIP_TRY(hipMemsetAsync(b.p, 0, want, st));
     return 0;
 }
 
@@ -411,8 +416,7 @@ extern "C" int smol_attn_ctx_destroy(smol_attn_ctx *ctx) {
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
     DevBuf *bufs[] = {&ctx->desc, &ctx->work, &ctx->out32, &ctx->dec_part};
-    for (DevBuf *b : bufs)
-        if (b->p) hipFree(b->p);
+    for (DevBuf *b : bufs) dev_free(*b);
     if (ctx->range_flag) hipHostFree(ctx->range_flag);
     if (ctx->mark) hipEventDestroy(ctx->mark);
     for (auto &s : ctx->ring) {

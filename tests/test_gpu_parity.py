@@ -692,6 +692,53 @@ def test_first_prefill_of_a_context(sa):
     assert fb <= 4 * fa
 
 
+def test_workspace_grows_under_calls_in_flight(sa):
+    """Calls of growing size enqueued with no wait between them: each one's
+    workspace replaces a smaller one that the kernels before it still read. The
+    bits are those of a context of their own."""
+    from smol_genius_amd.workloads import Prefill
+    print("workspace growth", flush=True)
+    sizes = [(40, 0), (130, 31), (300, 500), (700, 1000), (90, 3000), (1500, 2000)]
+    wls = [Prefill("t", 16, 8, 128, P, S, 1e6, seed=770 + i, in_bf16=False) for i, (S, P) in enumerate(sizes)]
+    xs = [{k: dev(v, k.startswith("cache")) for k, v in wl.inputs().items()} for wl in wls]
+    torch.cuda.synchronize()
+
+    def prepare(c, wl, x):
+        kv = sa.KVCache(c, 1, 1, wl.Hkv, wl.hd, wl.pos0 + wl.seq_q)
+        if wl.pos0:
+            kv.write(0, 0, 0, x["cache_k"], x["cache_v"])
+        rope = sa.RopeTable(c, wl.hd, wl.theta, 0, wl.pos0 + wl.seq_q)
+        return kv, rope, sa.prefill_call(c, kv, 0, 0, rope, wl.pos0, x["q"], x["k"], x["v"], wl.Hq, wl.scale)
+
+    want = []
+    for wl, x in zip(wls, xs):
+        c = sa.Context(0)
+        kv, rope, call = prepare(c, wl, x)
+        call()
+        c.synchronize()
+        want.append(call.out.cpu())
+        kv.close()
+        rope.close()
+        c.close()
+    c = sa.Context(0)
+    try:
+        calls = [prepare(c, wl, x) for wl, x in zip(wls, xs)]
+        for _ in range(2):
+            for _, _, call in calls:
+                call.out.zero_()
+            torch.cuda.synchronize()
+            for _, _, call in calls:
+                call()
+            c.synchronize()
+            for (_, _, call), w in zip(calls, want):
+                assert torch.equal(call.out.cpu(), w)
+        for kv, rope, _ in calls:
+            kv.close()
+            rope.close()
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("window,cap", [(16, 0.0), (0, 2.0), (1, 0.0), (40, 1.5), (1, 3.0)])
 def test_decode_window_softcap(ctx, sa, oracle, wo, window, cap):
     """Sliding window and softcap on decode (the new key is scored apart
