@@ -354,7 +354,6 @@ __device__ __forceinline__ void dma_1k(rsrc_t r, unsigned voff, unsigned soff, u
 }
 #pragma clang diagnostic pop
 
-#define SK_WAVES 4
 
 /* fp16 hi + lo of two floats (the probabilities of the precise P.V):
  * hi = fp16_rne(p), lo = fp16_rne(p - hi). p - hi is exact in fp32 (hi is p

@@ -213,7 +213,7 @@ typedef struct {
 #define DEC_ARG_ITEMS 320     /* workgroup items passed in the kernel arguments */
 #define DEC_SPIN_LIMIT (1 << 22) /* flag polls before a merger gives up (writes NaN rows and raises
                                     the context's merge flag) */
-#define SMOL_FLAG_WORDS 64       /* ints of a context's device flag block (256 bytes) */
+#define SMOL_FLAG_WORDS 64       /* ints of a context's flags (256 bytes of pinned host memory) */
 #define SMOL_FLAG_MERGE 32       /* word of the merge flag: its own 128-byte line */
 
 /* one workgroup of the grid (index = blockIdx.x); seq < 0: nothing to do.

@@ -1,7 +1,7 @@
 /*
  * gemm_device.h - what the GEMM kernels share (gemm.hip, gemm_rs.hip,
- * gemm_sw.hip): the tile of a workgroup, the split of fp32 rows into bf16 hi + lo, and the
- * fused operations at a tile's end.
+ * gemm_sw.hip): the tile of a workgroup, the split of fp32 rows into bf16
+ * hi + lo, and the fused operations at a tile's end.
  */
 #ifndef SMOL_GEMM_DEVICE_H
 #define SMOL_GEMM_DEVICE_H

@@ -10,9 +10,8 @@
  * once, on the way into LDS, by the thread that loaded them: 51.2 -> 47.5 us
  * there, 180 -> 162 us for 2048 -> 12288. (The norm's squares in eight parts a
  * row take 46.4 and 159 us, but leave the scale other last bits than the other
- * tiles' four.) (The smaller tiles and a bf16 x gain
- * nothing: 128 x 128 25.3 / 25.4 us, bf16 192 x 192 37.2 / 39.9; k_gemm's
- * direct transfers stay there. A third LDS stage, with the next step's
+ * tiles' four.) (128 x 128 and a bf16 x gain nothing: 25.3 / 25.4 us, bf16
+ * 192 x 192 37.2 / 39.9; k_gemm's direct transfers stay there. A third LDS stage, with the next step's
  * fragments read during the products, spilled registers: 58 us.)
  */
 #include "gemm_device.h"

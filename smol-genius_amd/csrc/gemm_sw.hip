@@ -286,7 +286,7 @@ extern "C" int smol_launch_gemm_sw(const GemmParams *p, int cfg, bool xbf, bool 
     case 4: return launch_sw<32, 64, 2, 2, 8, 128, 3, 128, 3, 8, 128, 3>(*p, xbf, ybf, st, e0, e1);
     case 5: return launch_sw<32, 32, 2, 2, 8, 256, 2, 128, 3, 8, 256, 2>(*p, xbf, ybf, st, e0, e1);
     case 6: return launch_sw<16, 32, 2, 1, 8, 256, 3, 256, 3, 8, 256, 3>(*p, xbf, ybf, st, e0, e1);
-    case 7: return launch_sw<16, 16, 1, 1, 8, 256, 4, 256, 4, 8, 256, 4>(*p, xbf, ybf, st, e0, e1);
+    case 7: return launch_sw<16, 16, 1, 1, 8, 256, 3, 256, 3, 8, 256, 3>(*p, xbf, ybf, st, e0, e1);
     default: return -1;
     }
 }

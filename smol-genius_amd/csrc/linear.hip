@@ -738,22 +738,22 @@ int run_gemv_rows(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const v
  * K in thousands. The constants are fitted (least squares of the relative
  * error) to the measured times of every configuration at 5 to 2048 rows, 640 to
  * 12288 outputs and K = 640 to 6144, weights not in L2, for a plain fp32 x, one
- * with the norm and a bf16 x; over those 484 products the choice is within 0.8%
- * of the best configuration on average, 26% at worst (1300 bf16 rows, 6144 ->
- * 2048: 83.2 us against 65.8). The bits are the same in every one of them.
- * Where the lines fall (rows up to which a k_gemm_sw tile is chosen): N = 1024,
- * K = 1024 to 3072: 2048 and more; N = 6144, K = 1024: 320; N = 12288, K = 2048
- * with the norm: 128. */
+ * with the norm and a bf16 x; over those 484 products the choice is within 0.6%
+ * of the best configuration on average, 26% at worst (700 bf16 rows, 1024 ->
+ * 6144: 34.2 us against 27.2, where 64 x 64 tiles share a compute unit). The
+ * bits are the same in every one of them. Where the lines fall (rows up to
+ * which a k_gemm_sw tile is chosen): N = 1024, K = 1024 to 3072: 2048 and more;
+ * N = 6144, K = 1024: 320; N = 12288, K = 2048 with the norm: 128. */
 int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, bool norm, int seg_align = 0) {
     static const float cost[GEMM_CFGS][3][4] = {
-        {{0.0f, 7.81f, 25.9f, 0.0444f}, {0.0f, 9.65f, 27.7f, 0.162f}, {0.0f, 6.44f, 17.1f, 0.0f}},
-        {{0.0f, 3.45f, 14.9f, 0.145f}, {0.0f, 5.34f, 17.8f, 0.0385f}, {0.0f, 5.27f, 10.5f, 0.00143f}},
-        {{4.29f, 0.0f, 5.44f, 0.0669f}, {2.23f, 2.86f, 7.52f, 0.0f}, {3.85f, 1.18f, 3.48f, 0.0108f}},
-        {{0.0f, 3.99f, 8.93f, 0.0779f}, {0.0f, 5.94f, 10.2f, 0.0257f}, {0.871f, 5.58f, 5.78f, 0.0f}},
-        {{1.87f, 2.09f, 3.61f, 0.0f}, {1.83f, 3.1f, 4.32f, 0.0104f}, {3.74f, 1.14f, 2.26f, 0.0214f}},
-        {{1.61f, 1.98f, 2.71f, 0.0f}, {2.59f, 2.01f, 3.61f, 0.0f}, {3.41f, 0.987f, 1.4f, 0.0243f}},
-        {{2.17f, 1.68f, 1.76f, 0.0f}, {2.04f, 3.01f, 1.91f, 0.0117f}, {3.51f, 0.751f, 1.01f, 0.0302f}},
-        {{3.14f, 0.951f, 1.27f, 0.0261f}, {2.47f, 2.59f, 1.59f, 0.00759f}, {3.33f, 0.897f, 0.732f, 0.027f}},
+        {{8.04f, 0.0f, 25.8f, 0.0629f}, {0.0f, 10.8f, 26.9f, 0.175f}, {0.0f, 5.94f, 17.4f, 0.0f}},
+        {{0.0f, 3.46f, 15.0f, 0.155f}, {0.0f, 5.33f, 17.8f, 0.0434f}, {0.0f, 4.53f, 10.9f, 0.0f}},
+        {{3.97f, 0.0f, 5.54f, 0.0655f}, {1.8f, 3.04f, 7.49f, 0.00561f}, {3.37f, 1.22f, 3.53f, 0.00749f}},
+        {{0.0f, 3.82f, 9.0f, 0.0906f}, {0.0f, 5.5f, 10.5f, 0.0256f}, {0.25f, 5.61f, 5.95f, 0.0f}},
+        {{1.26f, 2.35f, 3.64f, 0.0f}, {1.54f, 3.21f, 4.33f, 0.00732f}, {3.29f, 1.14f, 2.29f, 0.0204f}},
+        {{1.05f, 2.21f, 2.69f, 0.0f}, {2.27f, 2.05f, 3.66f, 0.0f}, {3.0f, 0.991f, 1.43f, 0.0162f}},
+        {{1.72f, 1.78f, 1.76f, 0.0f}, {1.75f, 3.09f, 1.92f, 0.00755f}, {3.01f, 0.761f, 1.02f, 0.0327f}},
+        {{2.68f, 0.92f, 1.27f, 0.0197f}, {2.13f, 2.49f, 1.65f, 0.00555f}, {2.75f, 0.917f, 0.726f, 0.0245f}},
     };
     const int forced = smol_internal_ctx_option(ctx, SMOL_OPT_GEMM_TILE);
     if (forced >= 1 && forced <= GEMM_CFGS) {
