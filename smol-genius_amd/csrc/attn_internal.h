@@ -57,6 +57,7 @@ typedef struct {
     int key_end;
     int n_split;     /* items of the row tile (its merge group) */
     int fresh_off;   /* the batch's fresh_row0 - fresh_pos0: fresh row of key k is k + fresh_off */
+    int pad0, pad1;  /* 32 bytes */
 } SkItem;
 
 /* An item with its batch, loaded together (the kernels issue one round of
@@ -76,7 +77,7 @@ typedef struct {
     int key_begin, key_end, fresh_off, row0;
     int n_rows, q_row0, out_tok0, q_pos0;
     int key_lo, key_hi, causal, next;
-    int n_split, part;
+    int n_split, part, pad0, pad1; /* 64 bytes: one aligned scalar load */
 } FbItem;
 
 /* A row tile whose keys were split over several items (k_sk_merge): its
