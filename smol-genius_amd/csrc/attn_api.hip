@@ -354,7 +354,7 @@ static int upload_desc(smol_attn_ctx *ctx, const void *host, size_t bytes) {
  * splits (Qwen3-0.6B sizes, 1025 keys: 19.8 us a layer, 12.3 with them). A
  * probe grid records each workgroup's XCC id (in `ids`, pinned host memory:
  * the context's flags, which it needs anyway; an allocation and a copy of the
- * probe's own made creation 66 us instead of XX); when one differs from its
+ * probe's own made creation 66 us instead of 44); when one differs from its
  * class, k_dec keeps every group in one workgroup. */
 #define XCD_PROBES 64 /* workgroups a class */
 static int check_xcd_dispatch(smol_attn_ctx *c, unsigned *ids) {
