@@ -91,6 +91,26 @@ __device__ __forceinline__ void split_frag(const float *v, b8 &hi, b8 &lo) {
     lo = as_b8(make_uint4(lw[0], lw[1], lw[2], lw[3]));
 }
 
+/* A row's sum of squares over 64-wide steps, eight lanes a row (lane lq holds
+ * chunk lq, eight values), in k_gemm's order: four running sums, of chunks q and
+ * then q + 4, which rest in lanes lq < 4, go to lanes lq + 4 and come back; at
+ * the end they are added as row_sum4 does (every lane lq < 4 gets the row's) */
+__device__ __forceinline__ float gemm_squares64(const float *v, float ss) {
+    auto squares = [&](float t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < 8; b++) t = fmaf(v[b], v[b], t);
+        return t;
+    };
+    const float up = __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(squares(ss)),
+                                                                 0x114 /* row_shr:4 */, 0xf, 0xf, true));
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(squares(up)), 0x104 /* row_shl:4 */, 0xf,
+                                                       0xf, true));
+}
+__device__ __forceinline__ float gemm_squares64_sum(float t) {
+    t += __shfl_xor(t, 2, 64);
+    return t + __shfl_xor(t, 1, 64);
+}
+
 /* v truncated to bf16, and the bf16 decoder's GeGLU of a truncated (gate, up)
  * pair before its own truncation: every step rounded as written
  * (qkn_bf16_decoder.c:235-251) */

@@ -100,17 +100,7 @@ void k_gemm_rs(const GemmParams p) {
             float v[8] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w),
                           __uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
             if constexpr (NORM) {
-                /* the row's four running sums (chunks lq, then lq + 4: k_gemm's
-                 * order) rest in lanes lq < 4, go to lanes lq + 4 and come back */
-                auto squares = [&](float t) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int b = 0; b < 8; b++) t = fmaf(v[b], v[b], t);
-                    return t;
-                };
-                const float up = __uint_as_float(__builtin_amdgcn_update_dpp(
-                    0, __float_as_uint(squares(ss[e])), 0x114 /* row_shr:4 */, 0xf, 0xf, true));
-                ss[e] = __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(squares(up)),
-                                                                    0x104 /* row_shl:4 */, 0xf, 0xf, true));
+                ss[e] = gemm_squares64(v, ss[e]);
                 const uint4 g0 = r.g[0], g1 = r.g[1];
                 const uint32_t g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
@@ -176,14 +166,11 @@ void k_gemm_rs(const GemmParams p) {
             __syncthreads();
         }
 
-    /* the rows' scale: threads 8 r .. 8 r + 3 hold row r's partial sums, added
-     * as row_sum4 does */
+    /* the rows' scale */
     if constexpr (NORM) {
 #pragma unroll
         for (int e = 0; e < XL; e++) {
-            float t = ss[e];
-            t += __shfl_xor(t, 2, 64);
-            t += __shfl_xor(t, 1, 64);
+            const float t = gemm_squares64_sum(ss[e]);
             if (lq == 0) s_rinv[lr + TPB / 8 * e] = 1.0f / sqrtf(t / (float)K + p.eps);
         }
         __syncthreads();

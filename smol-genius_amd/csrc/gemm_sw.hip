@@ -18,7 +18,9 @@
  * neighbouring lanes along a row) into registers, DEPTH slabs ahead, an fp32
  * x is split (and scaled) there, and goes into one of two LDS stages. WN x WM
  * waves multiply the other stage meanwhile, and with the norm BM / 16 more sum
- * the rows' squares. One barrier a slab. (With every wave doing both, the
+ * the rows' squares (in 64-wide slabs the staging threads: x as loaded in LDS
+ * too makes 64 x 64 21.2 us of 20.2, 64 rows, 2048 -> 12288, and 96 of 77, 1536
+ * rows, 1024 -> 6144). One barrier a slab. (With every wave doing both, the
  * multiplying waves' own staging delayed every slab: 26 fp32 rows, 6144 ->
  * 2048, 15.7 us.)
  *
@@ -35,8 +37,11 @@
  */
 #include "gemm_device.h"
 
+/* waves that sum squares: none with 64-wide slabs, where the staging threads do */
+constexpr int sw_square_waves(int bm, int kc, bool norm) { return norm && kc > 64 ? bm / 16 : 0; }
+
 template <int BM, int BN, int WN, int WM, int SW, int KC, int DEPTH, bool XBF, bool YBF, bool NORM>
-__global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_gemm_sw(const GemmParams p) {
+__global__ __launch_bounds__(64 * (SW + WN * WM + sw_square_waves(BM, KC, NORM))) void k_gemm_sw(const GemmParams p) {
     constexpr int TPB = 64 * SW, MW = WN * WM;
     constexpr int TN = BN / WN, TM = BM / WM, NT = TN / 16, MT = TM / 16; /* a multiplying wave's tile */
     constexpr int KS = KC / 32;   /* 32-wide steps of a slab */
@@ -44,16 +49,18 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
     constexpr int ROWB = KC * 2;  /* bytes of an LDS row */
     constexpr int RS = TPB / CPR; /* rows between two chunks of a staging thread */
     constexpr int SWZ = CPR < 16 ? 7 : 15; /* row bits that swizzle a chunk: a fragment's rows then span every bank */
-    /* a stage: W, x (hi), x lo, and with the norm x as loaded (the first four
-     * values of each chunk, then the last four) */
+    /* a stage: W, x (hi), x lo, and for waves that sum squares x as loaded (the
+     * first four values of each chunk, then the last four) */
+    constexpr bool RAW = sw_square_waves(BM, KC, NORM) > 0;
     constexpr int XH = BN * ROWB, XLO = XH + BM * ROWB, XR = XLO + (XBF ? 0 : BM * ROWB);
-    constexpr int STAGE = XR + (NORM ? 2 * BM * ROWB : 0);
+    constexpr int STAGE = XR + (RAW ? 2 * BM * ROWB : 0);
     constexpr int WL = BN * CPR / TPB, XL = BM * CPR / TPB; /* chunks a thread stages of W and x */
     static_assert(2 * STAGE <= 160 * 1024, "LDS");
     static_assert(WL * TPB == BN * CPR && XL * TPB == BM * CPR, "staging shape");
     static_assert(RS % (SWZ + 1) == 0, "every row of a thread has one swizzle");
     static_assert(KS % 2 == 0, "fragments are read two steps at a time");
     static_assert(!(XBF && NORM), "the norm takes an fp32 x");
+    static_assert(!NORM || RAW || KC == 64, "two 32-wide halves a slab");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * STAGE];
     float *const s_rinv = reinterpret_cast<float *>(smem); /* after the last slab */
 
@@ -110,6 +117,9 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
 #pragma unroll
             for (int e = 0; e < WL; e++) r.w[e] = bload(rw, w_off[e], (unsigned)(k0 * 2));
         };
+        float ss[XL];
+#pragma unroll
+        for (int e = 0; e < XL; e++) ss[e] = 0.0f;
         auto store = [&](const Raw &r, unsigned char *st) __attribute__((always_inline)) {
 #pragma unroll
             for (int e = 0; e < WL; e++) *reinterpret_cast<uint4 *>(st + pos + RS * e * ROWB) = r.w[e];
@@ -123,9 +133,13 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
                     float v[8] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z),
                                   __uint_as_float(u.w), __uint_as_float(w.x), __uint_as_float(w.y),
                                   __uint_as_float(w.z), __uint_as_float(w.w)};
-                    if constexpr (NORM) {
+                    if constexpr (RAW) {
                         *reinterpret_cast<uint4 *>(xp + XR) = u;
                         *reinterpret_cast<uint4 *>(xp + XR + BM * ROWB) = w;
+                    } else if constexpr (NORM) {
+                        ss[e] = gemm_squares64(v, ss[e]);
+                    }
+                    if constexpr (NORM) {
                         const uint4 g0 = r.g[0], g1 = r.g[1];
                         const uint32_t g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
@@ -154,6 +168,13 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
                 issue(s0 + u + 1 + DEPTH, raw[(u + 1) % DEPTH]);
                 __syncthreads();
             }
+        if constexpr (NORM && !RAW) {
+#pragma unroll
+            for (int e = 0; e < XL; e++) {
+                const float t = gemm_squares64_sum(ss[e]);
+                if (lq == 0) s_rinv[lr + RS * e] = 1.0f / sqrtf(t / (float)K + p.eps);
+            }
+        }
         if constexpr (NORM) __syncthreads();
         return;
     }
@@ -162,7 +183,7 @@ __global__ __launch_bounds__(64 * (SW + WN * WM + (NORM ? BM / 16 : 0))) void k_
     auto frag = [&](const unsigned char *base, int row, int ks) __attribute__((always_inline)) {
         return *reinterpret_cast<const uint4 *>(base + row * ROWB + (((4 * ks + j) ^ (row & SWZ)) << 4));
     };
-    if (NORM && wave >= SW + MW) {
+    if (RAW && wave >= SW + MW) {
         const int row = 16 * (wave - SW - MW) + c;
         float t = 0.0f;
         __syncthreads();
@@ -266,7 +287,7 @@ static int launch_sw(const GemmParams &p, bool xbf, bool ybf, hipStream_t st, hi
         if (ybf) hipExtLaunchKernelGGL((k_gemm_sw<BM, BN, WN, WM, SWB, KB, DB, true, true, false>), grid, block, 0, st, e0, e1, 0, p);
         else hipExtLaunchKernelGGL((k_gemm_sw<BM, BN, WN, WM, SWB, KB, DB, true, false, false>), grid, block, 0, st, e0, e1, 0, p);
     } else if (p.g) {
-        const dim3 block(64 * (SWF + MW + BM / 16));
+        const dim3 block(64 * (SWF + MW + sw_square_waves(BM, KN, true)));
         if (ybf) hipExtLaunchKernelGGL((k_gemm_sw<BM, BN, WN, WM, SWF, KN, DN, false, true, true>), grid, block, 0, st, e0, e1, 0, p);
         else hipExtLaunchKernelGGL((k_gemm_sw<BM, BN, WN, WM, SWF, KN, DN, false, false, true>), grid, block, 0, st, e0, e1, 0, p);
     } else {
@@ -282,7 +303,7 @@ extern "C" int smol_launch_gemm_sw(const GemmParams *p, int cfg, bool xbf, bool 
                                    hipEvent_t e1) {
     switch (cfg) {
     case 2: return launch_sw<64, 64, 2, 2, 8, 64, 4, 64, 3, 4, 64, 3>(*p, xbf, ybf, st, e0, e1);
-    case 3: return launch_sw<64, 128, 2, 2, 8, 64, 2, 64, 2, 8, 64, 3>(*p, xbf, ybf, st, e0, e1);
+    case 3: return launch_sw<64, 128, 2, 2, 8, 64, 2, 64, 3, 8, 64, 3>(*p, xbf, ybf, st, e0, e1);
     case 4: return launch_sw<32, 64, 2, 2, 8, 128, 3, 128, 3, 8, 128, 3>(*p, xbf, ybf, st, e0, e1);
     case 5: return launch_sw<32, 32, 2, 2, 8, 256, 2, 128, 3, 8, 256, 2>(*p, xbf, ybf, st, e0, e1);
     case 6: return launch_sw<16, 32, 2, 1, 8, 256, 3, 256, 3, 8, 256, 3>(*p, xbf, ybf, st, e0, e1);

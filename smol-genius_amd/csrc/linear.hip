@@ -738,22 +738,22 @@ int run_gemv_rows(smol_attn_ctx *ctx, hipStream_t st, void *y, bool ybf, const v
  * K in thousands. The constants are fitted (least squares of the relative
  * error) to the measured times of every configuration at 5 to 2048 rows, 640 to
  * 12288 outputs and K = 640 to 6144, weights not in L2, for a plain fp32 x, one
- * with the norm and a bf16 x; over those 484 products the choice is within 0.6%
- * of the best configuration on average, 26% at worst (700 bf16 rows, 1024 ->
- * 6144: 34.2 us against 27.2, where 64 x 64 tiles share a compute unit). The
+ * with the norm and a bf16 x; over those 484 products the choice is within 0.5%
+ * of the best configuration on average, 24% at worst (700 bf16 rows, 1024 ->
+ * 6144: 34.2 us against 27.5, where 64 x 64 tiles share a compute unit). The
  * bits are the same in every one of them. Where the lines fall (rows up to
  * which a k_gemm_sw tile is chosen): N = 1024, K = 1024 to 3072: 2048 and more;
  * N = 6144, K = 1024: 320; N = 12288, K = 2048 with the norm: 128. */
 int gemm_cfg(smol_attn_ctx *ctx, int M, int N, int K, bool xbf, bool norm, int seg_align = 0) {
     static const float cost[GEMM_CFGS][3][4] = {
-        {{8.04f, 0.0f, 25.8f, 0.0629f}, {0.0f, 10.8f, 26.9f, 0.175f}, {0.0f, 5.94f, 17.4f, 0.0f}},
-        {{0.0f, 3.46f, 15.0f, 0.155f}, {0.0f, 5.33f, 17.8f, 0.0434f}, {0.0f, 4.53f, 10.9f, 0.0f}},
-        {{3.97f, 0.0f, 5.54f, 0.0655f}, {1.8f, 3.04f, 7.49f, 0.00561f}, {3.37f, 1.22f, 3.53f, 0.00749f}},
-        {{0.0f, 3.82f, 9.0f, 0.0906f}, {0.0f, 5.5f, 10.5f, 0.0256f}, {0.25f, 5.61f, 5.95f, 0.0f}},
-        {{1.26f, 2.35f, 3.64f, 0.0f}, {1.54f, 3.21f, 4.33f, 0.00732f}, {3.29f, 1.14f, 2.29f, 0.0204f}},
-        {{1.05f, 2.21f, 2.69f, 0.0f}, {2.27f, 2.05f, 3.66f, 0.0f}, {3.0f, 0.991f, 1.43f, 0.0162f}},
-        {{1.72f, 1.78f, 1.76f, 0.0f}, {1.75f, 3.09f, 1.92f, 0.00755f}, {3.01f, 0.761f, 1.02f, 0.0327f}},
-        {{2.68f, 0.92f, 1.27f, 0.0197f}, {2.13f, 2.49f, 1.65f, 0.00555f}, {2.75f, 0.917f, 0.726f, 0.0245f}},
+        {{0.0f, 7.9f, 25.8f, 0.07f}, {0.0f, 11.0f, 26.9f, 0.163f}, {0.0f, 5.61f, 17.6f, 0.0f}},
+        {{0.0f, 3.32f, 15.0f, 0.141f}, {0.0f, 5.24f, 17.9f, 0.0424f}, {0.0f, 4.16f, 11.2f, 0.0f}},
+        {{3.7f, 0.0f, 5.63f, 0.0559f}, {3.38f, 1.74f, 6.37f, 0.0278f}, {3.13f, 1.27f, 3.54f, 0.0105f}},
+        {{0.0f, 3.69f, 9.08f, 0.0899f}, {0.336f, 5.41f, 9.15f, 0.0397f}, {0.0f, 5.66f, 6.0f, 0.0f}},
+        {{1.22f, 2.27f, 3.69f, 0.0f}, {1.39f, 3.23f, 4.34f, 0.00666f}, {3.08f, 1.18f, 2.3f, 0.0225f}},
+        {{1.06f, 2.2f, 2.69f, 0.0f}, {2.08f, 2.11f, 3.62f, 0.00256f}, {2.81f, 1.01f, 1.44f, 0.0161f}},
+        {{1.76f, 1.76f, 1.77f, 0.0f}, {1.58f, 3.1f, 1.89f, 0.0159f}, {2.84f, 0.779f, 1.02f, 0.0328f}},
+        {{2.74f, 0.933f, 1.26f, 0.00897f}, {2.02f, 2.48f, 1.66f, 0.00925f}, {2.57f, 0.925f, 0.726f, 0.0239f}},
     };
     const int forced = smol_internal_ctx_option(ctx, SMOL_OPT_GEMM_TILE);
     if (forced >= 1 && forced <= GEMM_CFGS) {
